@@ -27,7 +27,8 @@
 //                      (matvec_batch<..., BEPI_QKV>, batch.metal:94-165); with
 //                      qkv_small_kernel (up to 16 rows) and qkv_mid_kernel
 //                      (17..64 rows), the same arithmetic at every row count
-//   attn_rows_kernel   contiguous f32 attention (Kernels::attention)
+//   attn_rows_kernel   contiguous f32 attention (Kernels::attention), one row
+//                      per workgroup; attn_rows_tile_kernel: 16 rows, matrix cores
 //
 // Decode is HBM-bound streaming of f16 (or int8) K/V.  Arithmetic is f32 (the
 // matrix-core kernels carry f32 operands as f16 hi + lo parts); softmax runs
@@ -1931,6 +1932,260 @@ __device__ __forceinline__ void wait_tiles(uint32_t ahead) {
         __builtin_amdgcn_s_waitcnt(0x0f70);
 }
 
+// ------------------------------------- contiguous f32 attention, several rows
+
+// Kernels::attention for runs of queries, on the f32 matrix cores
+// (v_mfma_f32_16x16x4f32): a workgroup owns 16 consecutive queries of one head
+// and its W waves take 16-key tiles in turn, so no wave waits for another
+// before the merge at the end.  Per tile a wave computes S^T = K Q^T (the
+// online softmax runs on its columns, one query per lane column) and
+// O^T += V^T P^T, whose B operand is S^T's output registers as they are:
+// product j of PV takes keys 4g + j (g = lane / 16), the key the lane's score
+// j belongs to.
+//
+// K rows arrive by LDS DMA, whole rows, double-buffered per wave (no barrier):
+// the 16-byte piece c of row r sits at c ^ r, so the 16 lanes that read one
+// piece of 16 rows hit distinct banks.  V needs no LDS: a lane loads 4
+// consecutive dims of a row (16 lanes: 256 contiguous bytes), so O^T's row m
+// of product c is dim 4m + c and a lane ends up with 16 consecutive dims of
+// its query.
+//
+// Bound by the matrix cores and each tile's chain (QK, softmax, PV: ~1900
+// cycles of which 1024 are products): 1024 queries x 12 heads x 64 26 us
+// against 109 on attn_rows_kernel, where every query re-reads its keys.
+// 32 queries per wave (K/V read half as often, half the workgroups) took 28-34
+// us, all of K and V through LDS 27, more keys in flight (8 waves) 29.
+//
+// Error: the sums are cut so that it is that of attn_rows_kernel (1.3e-7 of
+// the result against 64 bits at 1024 keys; one accumulator throughout 2.6e-7):
+// a score adds D/4 products of 4 dims as a tree, and the keys go to 4
+// accumulators by key % 4.  The exponent reference follows the running max
+// only past kRefSlack (weights up to 2^8, f32 throughout).
+//
+// Rows past the last key repeat it (nothing past it is read).  A key hidden
+// from some query of a tile may hold infinities or NaN, which 0 * V would turn
+// into NaN in that query's sum: tiles with hidden keys check their V values
+// and, where one is not finite, add their rows one by one instead.
+constexpr int kRowsTile = 16;  // keys per tile, queries per workgroup
+
+template <int D, int W>
+__global__ __launch_bounds__(64 * W) void attn_rows_tile_kernel(const RowsLaunch a) {
+    constexpr int KC = D / 16;                  // 16-byte pieces of a K row per lane
+    constexpr int VG = D / 64;                  // 64-dim groups of V
+    constexpr int CH = D / 4;                   // 16-byte pieces per row
+    constexpr int RPL = 64 / CH;                // rows per DMA instruction
+    constexpr int NI = kRowsTile / RPL;         // DMA instructions per K tile
+    constexpr int NA = 4;                       // accumulators of PV
+    constexpr uint32_t TB = kRowsTile * D * 4;  // bytes of a K tile
+    constexpr size_t kTiles = (size_t)W * 2 * TB;
+    constexpr size_t kRed = (size_t)W * kRowsTile * (D + 2) * 4;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[kTiles > kRed ? kTiles : kRed];
+
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // Longest query blocks first.
+    const uint32_t n_qb = (a.n_q + kRowsTile - 1) / kRowsTile;
+    const uint32_t bi = blockIdx.x / a.n_head, h = blockIdx.x - bi * a.n_head;
+    const uint32_t q0 = (n_qb - 1 - bi) * kRowsTile;
+    const uint32_t nq = min(a.n_q - q0, (uint32_t)kRowsTile);
+    const uint32_t pos0 = a.q_pos0 + q0;  // position of the block's first query
+    const uint32_t n_kv = pos0 + nq;      // keys some query of the block sees
+    const uint32_t n_tiles = (n_kv + kRowsTile - 1) / kRowsTile;
+    const int col = lane & 15, rg = lane >> 4;
+
+    uint8_t* const my = lds + (size_t)wave * 2 * TB;  // [stage]
+    const uint32_t lds_my = (uint32_t)(uintptr_t)NI_LDS(my);
+    // A tile's rows lie at a scalar base plus a 32-bit byte offset per lane,
+    // the same for every tile but the last, whose rows past the last key
+    // repeat it (the launcher checks that 16 rows' strides fit).
+    const uint32_t dr = lane / CH, dc = lane % CH;  // this lane's row and piece within a DMA instruction
+    const uint32_t ks = (uint32_t)a.k_stride * 4, vs = (uint32_t)a.v_stride * 4;
+    uint32_t koff[NI];  // piece dc ^ r of row r = i * RPL + dr, to LDS piece dc of that row
+#pragma unroll
+    for (int i = 0; i < NI; i++) koff[i] = (i * RPL + dr) * ks + 16 * (dc ^ (i * RPL + dr));
+    const uint32_t voff = 4 * rg * vs + 16 * col;  // row 4rg, dims 4col ..
+    qkv_f4 vn[VG][4];  // the next tile's V: dims 64g + 4col .. +3 of key 4rg + j
+    auto issue = [&](uint32_t st, uint32_t t) {
+        const uint32_t j0 = t * kRowsTile;
+        const uint8_t* kb = reinterpret_cast<const uint8_t*>(a.k + (int64_t)j0 * a.k_stride + h * D);
+        const uint8_t* vb = reinterpret_cast<const uint8_t*>(a.v + (int64_t)j0 * a.v_stride + h * D);
+        if (j0 + kRowsTile <= n_kv) {
+#pragma unroll
+            for (int i = 0; i < NI; i++) lds_dma16_sbase(kb, koff[i], lds_my + st * TB + i * 1024);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int g = 0; g < VG; g++)
+                    vn[g][j] = *reinterpret_cast<const qkv_f4*>(vb + (uint32_t)j * vs + 256 * g + voff);
+        } else {
+            const uint32_t last = n_kv - 1 - j0;
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const uint32_t r = i * RPL + dr;
+                lds_dma16_sbase(kb, min(r, last) * ks + 16 * (dc ^ r), lds_my + st * TB + i * 1024);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t vo = min(4u * rg + j, last) * vs + 16 * col;
+#pragma unroll
+                for (int g = 0; g < VG; g++) vn[g][j] = *reinterpret_cast<const qkv_f4*>(vb + vo + 256 * g);
+            }
+        }
+    };
+    uint32_t t = wave;
+    if (t < n_tiles) issue(0, t);
+
+    // Q^T as the B operand: query col, dims 16u + 4rg .. +3.
+    qkv_f4 q[KC];
+    {
+        const bool has = (uint32_t)col < nq;
+        const float* qp = a.q + (int64_t)(q0 + (has ? col : 0)) * a.q_stride + h * D + 4 * rg;
+#pragma unroll
+        for (int u = 0; u < KC; u++) {
+            const qkv_f4 x = *reinterpret_cast<const qkv_f4*>(qp + 16 * u);
+#pragma unroll
+            for (int e = 0; e < 4; e++) q[u][e] = has ? x[e] * a.qscale : 0.f;
+        }
+    }
+    float m = kMinScore, l = 0.f;
+    float4_t o[NA][VG][4];
+#pragma unroll
+    for (int n = 0; n < NA; n++)
+#pragma unroll
+        for (int g = 0; g < VG; g++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) o[n][g][c] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    uint32_t st = 0;
+    for (; t < n_tiles; t += W) {
+        // This tile's V registers, and with them its K DMA, issued before them
+        // (loads land in order; the explicit wait is for the compiler's sake,
+        // which does not count the DMA).
+        qkv_f4 v[VG][4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int g = 0; g < VG; g++) {
+                asm volatile("" : "+v"(vn[g][j]) : : "memory");
+                v[g][j] = vn[g][j];
+            }
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        const uint8_t* const kt = my + st * TB;
+        st ^= 1;
+        const uint32_t j0 = t * kRowsTile;
+        qkv_f4 kv[KC];
+#pragma unroll
+        for (int u = 0; u < KC; u++)
+            kv[u] = *reinterpret_cast<const qkv_f4*>(kt + ((uint32_t)col * CH + ((4 * u + rg) ^ col)) * 16);
+        // The next tile goes to the other stage, whose reads (the previous
+        // tile's K) were waited for before that tile's products.
+        if (t + W < n_tiles) issue(st, t + W);
+        // Product e of piece u covers dims 16u + 4g + e (g = 0..3) in an
+        // accumulator of its own; the 4 * KC of them are added as a tree.
+        float4_t su[4 * KC];
+#pragma unroll
+        for (int u = 0; u < KC; u++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                su[4 * u + e] =
+                    __builtin_amdgcn_mfma_f32_16x16x4f32(kv[u][e], q[u][e], float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+        for (int w = 2 * KC; w > 0; w /= 2)
+#pragma unroll
+            for (int u = 0; u < w; u++) su[u] += su[u + w];
+        float4_t s = su[0];
+        const bool masked = j0 + kRowsTile - 1 > pos0;  // some key is hidden from some query
+        if (masked) {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (j0 + 4 * rg + e > pos0 + col) s[e] = -INFINITY;
+        }
+        const float lm = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+        if (__any(lm > m + kRefSlack)) {
+            const float mn = fmaxf(m, rows4_max(lm));
+            const float alpha = fast_exp2(m - mn);
+            m = mn;
+            l *= alpha;
+#pragma unroll
+            for (int n = 0; n < NA; n++)
+#pragma unroll
+                for (int g = 0; g < VG; g++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++) o[n][g][c] *= alpha;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) s[e] = fast_exp2(s[e] - m);
+        l += (s[0] + s[1]) + (s[2] + s[3]);
+        if (masked) {
+            bool bad = false;
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int g = 0; g < VG; g++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) bad |= (__float_as_uint(v[g][j][e]) & 0x7fffffffu) >= 0x7f800000u;
+            if (__any(bad)) {
+                const uint32_t n_keys = min((uint32_t)kRowsTile, n_kv - j0);
+#pragma unroll 1
+                for (uint32_t key = 0; key < n_keys; key++) {
+                    const float pj = key % 4 == 0 ? s[0] : key % 4 == 1 ? s[1] : key % 4 == 2 ? s[2] : s[3];
+                    const float p = __shfl(pj, (int)(key / 4) * 16 + col);
+                    if (j0 + key <= pos0 + col) {
+                        const float* vp = a.v + (int64_t)(j0 + key) * a.v_stride + h * D + 16 * rg;
+#pragma unroll
+                        for (int g = 0; g < VG; g++)
+#pragma unroll
+                            for (int e = 0; e < 4; e++)  // dims 64g + 16rg + 4e + c
+#pragma unroll
+                                for (int c = 0; c < 4; c++)
+                                    o[0][g][c][e] = fmaf(p, vp[64 * g + 4 * e + c], o[0][g][c][e]);
+                    }
+                }
+                continue;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int g = 0; g < VG; g++)
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    o[j][g][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[g][j][c], s[j], o[j][g][c], 0, 0, 0);
+    }
+    // Merge the waves' states through LDS, over the tiles.
+    __syncthreads();
+    auto& red = *reinterpret_cast<float(*)[W][kRowsTile][D + 2]>(lds);
+    l = rows4_sum(l);
+    float* const r = red[wave][col];
+    if (rg == 0) {
+        r[0] = m;
+        r[1] = l;
+    }
+#pragma unroll
+    for (int g = 0; g < VG; g++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float4_t x = (o[0][g][c] + o[1][g][c]) + (o[2][g][c] + o[3][g][c]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) r[2 + 64 * g + 16 * rg + 4 * e + c] = x[e];
+        }
+    __syncthreads();
+    for (uint32_t u = threadIdx.x; u < nq * D; u += 64 * W) {
+        const uint32_t row = u / D, d = u - row * D;
+        float M = red[0][row][0];
+#pragma unroll
+        for (int w = 1; w < W; w++) M = fmaxf(M, red[w][row][0]);
+        float L = 0.f, O = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const float wt = fast_exp2(red[w][row][0] - M);
+            L += red[w][row][1] * wt;
+            O += red[w][row][2 + d] * wt;
+        }
+        a.out[(int64_t)(q0 + row) * a.out_stride + h * D + d] = O / L;
+    }
+}
+
 // QKV projection of mid-size batches (kQkvSmallRows < n <= kQkvMidRows):
 // a workgroup of 8 waves owns a 16-row x 16-feature tile, as
 // qkv_small_kernel with one row block, but x and W reach the matrix cores
@@ -3247,16 +3502,51 @@ hipError_t launch_stream(bool copy, bool span, const void* src, void* dst, size_
     return hipGetLastError();
 }
 
+template <int D>
+hipError_t launch_attention_rows_t(const RowsLaunch& a, hipStream_t s) {
+    const uint64_t rows = (uint64_t)a.n_q * a.n_head;
+    const uint32_t cus = device_cus();
+    // Matrix-core tiles when their chain of 16-key tiles, ~(n_kv + 150) keys
+    // long counting the launch, costs less than the row kernel's work, whose
+    // every query reads its keys (12 heads x 64, row against tile kernel: 128
+    // queries of 128 keys 4.6 / 5.2 us, 256 of 256 11.4 / 6.9, 64 of 1064 18.2
+    // / 16.0, 1024 of 1024 109 / 26; 32 heads x 128: 16 of 1016 27.6 / 38, 32 of
+    // 1032 52 / 40, 250 of 250 49 / 20).  The tile kernel holds 16 rows'
+    // offsets in 32 bits.
+    const uint64_t n_kv = (uint64_t)a.q_pos0 + a.n_q;
+    const uint64_t keys = (uint64_t)a.n_q * a.q_pos0 + (uint64_t)a.n_q * (a.n_q + 1) / 2;
+    const int64_t max_stride = (int64_t)1 << 24;  // floats
+    if (a.k_stride <= max_stride && a.v_stride <= max_stride &&
+        (double)keys * a.n_head * D > (D == 64 ? 46000.0 : 66000.0) * (double)(n_kv + 150)) {
+        const uint32_t blocks = (a.n_q + kRowsTile - 1) / kRowsTile * a.n_head;
+        if constexpr (D == 64) {
+            // 8 waves while that leaves CUs half empty (384 workgroups: 11.6
+            // against 12.0 us; 48: 16.0 against 18.0; 608: 19.0 against 14.9).
+            if (blocks <= cus + cus / 2) {
+                hipLaunchKernelGGL((attn_rows_tile_kernel<D, 8>), dim3(blocks), dim3(512), 0, s, a);
+                return hipGetLastError();
+            }
+        }
+        hipLaunchKernelGGL((attn_rows_tile_kernel<D, 4>), dim3(blocks), dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
+    // Rows alone on their CUs take 8 waves (12 heads x 64, 1 query of 1001
+    // keys: 5.8 against 7.5 us, 16 of 1016 6.6 against 8.3, 32 of 1032 11.7
+    // against 11.3; 16 waves 6.2 for the first).
+    if (rows <= cus)
+        hipLaunchKernelGGL((attn_rows_kernel<D, 8>), dim3((uint32_t)rows), dim3(512), 0, s, a);
+    else
+        hipLaunchKernelGGL((attn_rows_kernel<D, 4>), dim3((uint32_t)rows), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_attention_rows(const RowsLaunch& a, hipStream_t s) {
-    const uint64_t blocks = (uint64_t)a.n_q * a.n_head;
-    if (blocks == 0) return hipSuccess;
-    constexpr int W = 4;
+    if ((uint64_t)a.n_q * a.n_head == 0) return hipSuccess;
     switch (a.head_dim) {
-        case 64: hipLaunchKernelGGL((attn_rows_kernel<64, W>), dim3((uint32_t)blocks), dim3(64 * W), 0, s, a); break;
-        case 128: hipLaunchKernelGGL((attn_rows_kernel<128, W>), dim3((uint32_t)blocks), dim3(64 * W), 0, s, a); break;
+        case 64: return launch_attention_rows_t<64>(a, s);
+        case 128: return launch_attention_rows_t<128>(a, s);
         default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_f32_to_f16(const float* in, uint16_t* out, size_t n, hipStream_t s) {
