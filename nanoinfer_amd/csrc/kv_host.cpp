@@ -38,9 +38,6 @@ constexpr uint32_t kRingSlots = 4;
 // Plans are uploaded on the handle's own copy stream and the caller's stream
 // waits for the upload with an event, so the copy overlaps the previous
 // step's kernels instead of sitting between them.
-// Query groups (matrix-core kernel) take wide workgroups from this many
-// (item, layer, head) units on, instead of splitting into partitions.
-constexpr uint64_t kWideMinGroupUnits = 256;
 // A step of prompt chunks (every sequence queried as prefill groups, no
 // partitions) on a Q8 pool with at least this many (sequence, layer, head)
 // units: the prefill launch appends each sequence's rows (one workgroup per
@@ -103,7 +100,7 @@ struct Plan {
     uint32_t nq_tile = 1;
     uint32_t napp_total = 0;  // fused: rows the attention items append
     bool fused = false;
-    bool wide = false;        // kWideWaves waves per attention workgroup
+    uint32_t wide = 0;        // waves per attention workgroup: AttnLaunch::wide
     bool seq_prefill = false; // every row belongs to a sequence queried as prefill groups (see pseqs)
     // Some launch of the plan reads the append entries `app` (an append
     // launch, a workgroup prologue, a prefill workgroup's appends); a fused
@@ -127,7 +124,7 @@ struct Plan {
         nq_tile = 1;
         napp_total = 0;
         fused = false;
-        wide = false;
+        wide = 0;
         app_read = true;
     }
 };
@@ -377,6 +374,9 @@ void balance_units(ni_kv* kv, Plan& P, uint32_t n_lay) {
     const uint64_t C = device_cus();
     const bool fused = P.napp_total > 0 || !P.orphans.empty();
     const uint64_t S = wide_blocks_per_cu(kv->o.head_dim, is_q8(kv->o), P.nq_tile, fused);
+    // (not for single rows of ni_kv_step_noalloc in launches this small: the
+    // order array would lower the size of step it takes)
+    if (kv->no_alloc && P.nq_tile == 1 && n_units < 512) return;
     // (one round: every block has a CU of its own already)
     if (S == 0 || n_units <= C || n_units > C * S || n_units > 65536) return;
     const uint64_t R = (n_units + C - 1) / C;  // rounds; CUs below `rem` receive R blocks, the others R - 1
@@ -458,11 +458,24 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
     // the tail is short -- only items longer than kLongItem keys are split
     // then.  Below that, the largest of 1024/512/256/128 tokens that yields
     // >= 2048 workgroups.
-    // Between kWideMinUnits and kFillWorkgroups units of single-row items
-    // (head_dim 64: a launch of one layer of 43..170 sequences), workgroups
-    // of kWideWaves waves share each item's pages instead of splitting it:
-    // no partials, no merge launch.  Query groups of up to one matrix tile
-    // (a verify step's rows) do the same from kWideMinGroupUnits units.
+    // At head_dim 64, launches of single rows or of groups within one matrix
+    // tile below that are not split either: several waves of one workgroup
+    // share each item's pages and merge in LDS, no partials, no merge launch
+    // (us per launch, split and merged against one workgroup per item):
+    // * single rows: kWideWaves waves (Q8: kWideWavesQ8), kSoloWaves while
+    //   every unit has a CU of its own and the items are long enough to keep
+    //   16 waves busy, kWaves up to kNarrowKeys keys, where waves of 2 pages
+    //   cover an item at once.  12 layers x 12 heads: 1 sequence of 150 keys
+    //   7.1 / 3.9, 300 7.9 / 5.2, 517 9.2 / 6.6, 1000 11.5 / 9.1, 3000 24.3 /
+    //   20.5, 3 of 1000 24.3 / 19.0; Q8 517 9.9 / 7.0, 3 of 1000 21.0 / 13.2.
+    // * groups: kWideWaves waves below kWideMinUnits units (12 layers, 5 rows of
+    //   300 keys 8.2 / 5.8, 1000 13.7 / 10.1), from there on, where two such
+    //   workgroups no longer fit each CU, kWaves (4 x U[64,1000] 23.2 -> 19.5,
+    //   13 41.9 -> 37.0).
+    // Below kWholeMinUnits units that holds up to kShortItem keys only: longer
+    // items fill the GPU faster in partitions (one layer of 12 heads: 1
+    // sequence of 2000 keys 8.1 / 12.5, 4 of 2000 11.4 / 13.4, 16 of 2000 24.1 /
+    // 18.8).
     // Prefill groups (more rows than one matrix tile, in a launch of their
     // own) are split automatically only past kLongItem keys: each of their
     // workgroups already carries 64 queries, and splitting them to fill the
@@ -476,11 +489,14 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
     if (part == 0) {
         constexpr uint64_t kFillWorkgroups = 2048;
         constexpr uint64_t kWideMinUnits = 512;
+        constexpr uint64_t kWholeMinUnits = 96;
+        constexpr uint32_t kNarrowKeys = 128, kSoloKeys = 384, kSoloKeysQ8 = 640;
         static const uint32_t kChoices[] = {1024, 512, 256, 128};
         pre_part = kLongItem;
         const uint64_t per_unit = (uint64_t)n_lay * kv->o.n_head;
         const uint64_t units = (uint64_t)groups.size() * per_unit;
         constexpr uint32_t kShortItem = 1280;  // keys (a 1024-token context and its new rows)
+        const uint32_t whole_keys = units >= kWholeMinUnits ? kLongItem : kShortItem;
         bool single = true, tiles = true;  // every group one row; every group within one matrix tile
         uint32_t max_keys = 0;
         for (const Group& g : groups) {
@@ -490,9 +506,14 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
         }
         if (units >= kFillWorkgroups) {
             part = kLongItem;
-        } else if (tiles && units >= (single ? kWideMinUnits : kWideMinGroupUnits) && kv->o.head_dim == 64) {
+        } else if (tiles && kv->o.head_dim == 64 &&
+                   (units >= (single ? kWideMinUnits : kWideMinUnits / 2) || max_keys <= whole_keys)) {
             part = kLongItem;
-            P.wide = true;
+            const uint32_t solo_keys = is_q8(kv->o) ? kSoloKeysQ8 : kSoloKeys;
+            if (!single)
+                P.wide = units < kWideMinUnits ? 1u : 0u;
+            else if (units >= kWideMinUnits || max_keys > kNarrowKeys)
+                P.wide = units <= device_cus() && max_keys > solo_keys ? 2u : 1u;
         } else if (n_lay == 1 && max_keys <= kShortItem) {
             // One layer per launch and no item past kShortItem keys: the
             // merge launch a split needs costs more than the fill it buys
@@ -975,7 +996,7 @@ int run_placed(ni_kv* kv, const Plan& P, const Offsets& off, const PlanRef& ref,
         a.n_lay = n_lay;
         a.nq_tile = P.nq_tile;
         a.qscale = (float)(1.4426950408889634 / std::sqrt((double)D));
-        a.wide = P.wide ? 1u : 0u;
+        a.wide = P.wide;
         a.off_order = (uint32_t)off.order;
         a.ordered = P.order.empty() ? 0u : 1u;
         a.n_orphan_blocks = P.fused ? orphan_blocks(a) : 0;

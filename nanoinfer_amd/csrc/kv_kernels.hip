@@ -38,6 +38,7 @@
 
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "kv_plan.h"
@@ -874,14 +875,15 @@ __global__ __launch_bounds__(64 * W) void attn_q8_kernel(const AttnLaunch a, con
     const uint32_t pg_end = (it.kv_end + kPage - 1) / kPage;
     constexpr uint32_t STRIDE = W * PB;
 
-    // Fused, in the wide (one layer per launch) workgroups: the item's new
+    // Fused, in the wide workgroups: the item's new
     // rows come from the k/v input as their pages stream, quantised as the
     // append quantises them (the row's amax reduced over its LPK lanes; a max
     // does not depend on the order).  Otherwise they are appended first
     // (streaming them costs ~24 registers, 7 -> 5 waves per SIMD, which all
     // layers in one launch lose: 5202 against 4638 GB/s; one layer per
-    // launch gains, 2641 -> 2823).
-    constexpr bool STREAM = D == 64 && W == (int)kWideWavesQ8 && (int)kWideWavesQ8 != kWaves;
+    // launch gains, 2641 -> 2823).  Workgroups of 16 waves, alone on their
+    // CUs, stream them too.
+    constexpr bool STREAM = D == 64 && W != kWaves;
     NewRows nr{};
     if constexpr (FUSED) {
         if (it.napp) {
@@ -3142,16 +3144,17 @@ hipError_t attn_launch_t(const AttnLaunch& a, const void* ip, uint32_t ib, hipSt
     const uint64_t blocks = (uint64_t)a.n_items * a.n_lay * a.pool.n_head + a.n_orphan_blocks;
     if (blocks == 0) return hipSuccess;
     if constexpr (D == 64 && NQ == 1) {
-        if (a.wide) {
-            constexpr int WW = kWideWaves;
-            constexpr int WPB = kWidePages;
+        auto wide = [&](auto wc) {
+            constexpr int WW = decltype(wc)::value;
             return with_plan(a, ip, ib, [&](auto pa) {
                 constexpr int INL = sizeof(pa.b) > 4 ? (int)sizeof(pa.b) : 0;
                 if (a.napp_total || a.n_orphan_blocks)
-                    return go(attn_split_kernel<D, NQ, WW, WPB, true, INL>, blocks, 64 * WW, s, t, a, pa);
-                return go(attn_split_kernel<D, NQ, WW, WPB, false, INL>, blocks, 64 * WW, s, t, a, pa);
+                    return go(attn_split_kernel<D, NQ, WW, kWidePages, true, INL>, blocks, 64 * WW, s, t, a, pa);
+                return go(attn_split_kernel<D, NQ, WW, kWidePages, false, INL>, blocks, 64 * WW, s, t, a, pa);
             });
-        }
+        };
+        if (a.wide == 2) return wide(std::integral_constant<int, (int)kSoloWaves>{});
+        if (a.wide) return wide(std::integral_constant<int, (int)kWideWaves>{});
     }
     if (a.wide) return hipErrorInvalidValue;
     return with_plan(a, ip, ib, [&](auto pa) {
@@ -3177,7 +3180,7 @@ hipError_t mfma_launch_t(const AttnLaunch& a, const void* ip, uint32_t ib, hipSt
     const uint64_t blocks = (uint64_t)a.n_items * a.n_lay * a.pool.n_head + a.n_orphan_blocks;
     if (blocks == 0) return hipSuccess;
     if constexpr (D == 64) {
-        if (a.wide) {  // kWideWaves waves share each item's pages
+        if (a.wide == 1) {  // kWideWaves waves share each item's pages
             constexpr int WW = kWideWaves;
             return with_plan(a, ip, ib, [&](auto pa) {
                 constexpr int INL = sizeof(pa.b) > 4 ? (int)sizeof(pa.b) : 0;
@@ -3230,8 +3233,8 @@ hipError_t q8_launch_t(const AttnLaunch& a, const void* ip, uint32_t ib, hipStre
     const uint64_t blocks = (uint64_t)a.n_items * a.n_lay * a.pool.n_head + a.n_orphan_blocks;
     if (blocks == 0) return hipSuccess;
     if constexpr (D == 64) {
-        if (a.wide) {
-            constexpr int WW = kWideWavesQ8;
+        auto wide = [&](auto wc) {
+            constexpr int WW = decltype(wc)::value;
             return with_plan(a, ip, ib, [&](auto pa) {
                 constexpr int INL = sizeof(pa.b) > 4 ? (int)sizeof(pa.b) : 0;
                 constexpr int PB = kQ8Pages;
@@ -3239,7 +3242,9 @@ hipError_t q8_launch_t(const AttnLaunch& a, const void* ip, uint32_t ib, hipStre
                     return go(attn_q8_kernel<D, WW, PB, true, INL>, blocks, 64 * WW, s, t, a, pa);
                 return go(attn_q8_kernel<D, WW, PB, false, INL>, blocks, 64 * WW, s, t, a, pa);
             });
-        }
+        };
+        if (a.wide == 2) return wide(std::integral_constant<int, (int)kSoloWaves>{});
+        if (a.wide) return wide(std::integral_constant<int, (int)kWideWavesQ8>{});
     }
     if (a.wide) return hipErrorInvalidValue;
     return with_plan(a, ip, ib, [&](auto pa) {
@@ -3480,7 +3485,9 @@ uint32_t orphan_blocks(const AttnLaunch& a) {
     const uint64_t threads = (uint64_t)a.n_lay * a.n_orphans * 2 * ((a.pool.n_head * a.pool.head_dim) >> 3);
     // Threads per workgroup of the launch the orphan blocks join.
     const bool q8_rows = a.pool.q8 && a.nq_tile == 1;
-    const uint64_t per_block = 64ull * (a.wide ? (q8_rows ? kWideWavesQ8 : kWideWaves) : kWaves);
+    const uint64_t per_block = 64ull * (a.wide == 2 ? kSoloWaves
+                                        : a.wide    ? (q8_rows ? kWideWavesQ8 : kWideWaves)
+                                                    : (uint32_t)kWaves);
     return (uint32_t)((threads + per_block - 1) / per_block);
 }
 

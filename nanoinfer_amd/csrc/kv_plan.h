@@ -30,6 +30,13 @@ constexpr uint32_t kWideWaves = 8;
 // The same for single rows on the Q8 cache (attn_q8_kernel), one layer per
 // launch config 3: 5 waves 2634 GB/s, 6 2602, 8 2444.
 constexpr uint32_t kWideWavesQ8 = 5;
+// Waves per workgroup of single rows when every (item, layer, head) unit has a
+// CU of its own: the unit's pages then come in at the CU's own rate, which
+// needs more of them in flight (one sequence of 517 keys, 12 layers x 12
+// heads: 8 waves 6.8 us, 16 6.6; of 1000 keys 10.1 and 9.1; 8 x U[64,1000],
+// one layer, 9.0 and 8.0; from two workgroups per CU on, 16 waves lose: 2 x
+// U[64,1000], 12 layers, 6.1 and 8.3).
+constexpr uint32_t kSoloWaves = 16;
 constexpr uint32_t kMaxGroupRows = kMfmaTile;  // most query rows sharing one K/V stream
 
 // Where one appended row goes: pool page `page`, position `slot` (0..15) in it.
@@ -215,7 +222,8 @@ struct AttnLaunch {
     uint32_t n_lay;
     uint32_t nq_tile;         // query tile: 1..8 (vector kernel), kMfmaTile (matrix cores) or kPrefillRows
     float qscale;             // log2(e) / sqrt(head_dim)
-    uint32_t wide;            // 1: kWideWaves waves per workgroup (single-row items, head_dim 64)
+    uint32_t wide;            // head_dim 64: 1: kWideWaves (rows on Q8: kWideWavesQ8) waves per workgroup,
+                              //   2: kSoloWaves (single rows)
     uint32_t off_pseqs;       // prefill launch: PrefillSeq[n_pseqs]; 0 sequences: one workgroup per item
     uint32_t n_pseqs;
     uint32_t merge_split;     // merge launch: the largest merge_split_of over its items (0 = 1)
