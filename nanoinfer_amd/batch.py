@@ -70,17 +70,79 @@ class BatchOpts:
         return self.n_head * self.head_dim
 
 
-def _stream_ptr(stream) -> int:
-    import torch
+# torch, its Tensor and float32, and the query of the current stream's handle
+# (None where this torch has none), set by _torch() on first use.  A call of one
+# layer has to cost the host less than its kernel: no import, no Stream object,
+# each property of a tensor asked for once (host time of a 12-layer step one
+# layer per call, 64 sequences, 222 -> 147 us; of one token's contiguous
+# attention 10.4 -> 6.9; of a layer's projection and attention 41 -> 32).
+_tc = _Tensor = _float32 = _raw_stream = _get_device = None
 
-    s = stream if stream is not None else torch.cuda.current_stream()
+
+def _torch():
+    global _tc, _Tensor, _float32, _raw_stream, _get_device
+    if _tc is None:
+        import torch
+
+        _Tensor, _float32 = torch.Tensor, torch.float32
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        _get_device = getattr(torch._C, "_cuda_getDevice", None)
+        _tc = torch
+    return _tc
+
+
+def _stream_ptr(stream) -> int:
+    if stream is None and _raw_stream is not None and _get_device is not None and _tc.cuda.is_initialized():
+        return _raw_stream(_get_device())
+    s = stream if stream is not None else _torch().cuda.current_stream()
     return int(s.cuda_stream)
+
+
+def _fits(t, rows, c, device):
+    """The row stride of a float32 tensor [>= rows, c] on the GPU `device` with
+    unit stride in its last dimension, or None: the quick form of _f32_arg and
+    _on_device, which say what is wrong with a tensor that does not fit."""
+    if type(t) is _Tensor and t.dtype is _float32 and t.is_cuda and t.get_device() == device:
+        shape = t.shape
+        if len(shape) == 2 and shape[0] >= rows and shape[1] == c:
+            stride = t.stride()
+            if stride[1] == 1:
+                return stride[0]
+    return None
+
+
+def _fits_layers(t, rows, c, n_layer, device):
+    """_fits for [n_layer, >= rows, c]: (row stride, layer stride) or None."""
+    if type(t) is _Tensor and t.dtype is _float32 and t.is_cuda and t.get_device() == device:
+        shape = t.shape
+        if len(shape) == 3 and shape[0] == n_layer and shape[1] >= rows and shape[2] == c:
+            stride = t.stride()
+            if stride[2] == 1:
+                return stride[1], stride[0]
+    return None
+
+
+def _fits_wide(t, rows, c, device) -> bool:
+    """Whether t is a float32 tensor [>= rows, >= c] on the GPU `device` with
+    unit stride in its last dimension."""
+    if type(t) is _Tensor and t.dtype is _float32 and t.is_cuda and t.get_device() == device:
+        shape = t.shape
+        return len(shape) == 2 and shape[0] >= rows and shape[1] >= c and t.stride(1) == 1
+    return False
+
+
+_no_rows, _no_work = _abi.ni_row * 0, _abi.ni_work * 0
+
+
+def _pointer(arr, empty, item):
+    """arr's data as a pointer to `item` (`empty`: its array type of no
+    elements, a view of a writable buffer in a sixth of the time of data_as)."""
+    return empty.from_buffer(arr) if arr.size and arr.flags.writeable else arr.ctypes.data_as(C.POINTER(item))
 
 
 def _rows(rows) -> tuple:
     arr = np.ascontiguousarray(np.asarray(rows, dtype=np.uint32).reshape(-1, 2))
-    n = arr.shape[0]
-    return arr, arr.ctypes.data_as(C.POINTER(_abi.ni_row)), n
+    return arr, _pointer(arr, _no_rows, _abi.ni_row), arr.shape[0]
 
 
 def _f32_arg(t, name, layered, rows, c, n_layer):
@@ -89,8 +151,7 @@ def _f32_arg(t, name, layered, rows, c, n_layer):
     dimension.  The C ABI sees only pointers and strides, so a short tensor is
     refused here, before any device access (`_on_device` checks placement
     once every layout has passed)."""
-    import torch
-
+    torch = _torch()
     if not isinstance(t, torch.Tensor) or t.dtype != torch.float32:
         raise TypeError(f"{name} must be a float32 CUDA tensor")
     if layered:
@@ -131,8 +192,7 @@ def _weights(w, bias, c, d_in, fmt="f32"):
     """Check the layout of W [3C, d_in] in format fmt (f32: a contiguous
     float32 [3C, d_in] tensor; otherwise a contiguous uint8 tensor of the
     format's bytes) and bias."""
-    import torch
-
+    torch = _torch()
     if fmt not in W_FORMATS:
         raise ValueError(f"unknown weight format {fmt!r} (one of {sorted(W_FORMATS)})")
     if fmt == "f32":
@@ -157,7 +217,7 @@ def _work(work) -> np.ndarray:
 
 def _work_rows(w: np.ndarray) -> int:
     """Rows a step's work numbers (sum of n_new)."""
-    return int(w[:, 1].astype(np.int64).sum())
+    return int(np.add.reduce(w[:, 1], dtype=np.int64))
 
 
 class PagedKv:
@@ -181,6 +241,7 @@ class PagedKv:
 
             self.device = torch.cuda.current_device()
         self._open_rows = None  # rows of the step opened by step_begin
+        self._c, self._n_layer = opts.n_embd, opts.n_layer
         h = C.c_void_p()
         rc = self._L.ni_kv_create(C.byref(o), C.byref(h))
         if rc != 0:
@@ -292,20 +353,26 @@ class PagedKv:
         the rows' page slots of `layer` as f16, q is returned [n, C].
         w_format "f16", "q8_0" or "q4_0": w holds the matrix in the
         reference's format (weights.rs:12-86), any dtype, contiguous."""
-        import torch
-
+        torch = _torch()
         arr, rp, n = _rows(rows)
         if not isinstance(x, torch.Tensor) or x.dim() != 2:
             raise ValueError("x must be a [rows, d_in] tensor")
-        xs, _ = self._f32(x, "x", False, n, c=x.shape[1])
-        _weights(w, bias, self.opts.n_embd, x.shape[1], w_format)
-        if q_out is not None:
-            self._f32(q_out, "q_out", False, n)
-        self._on_device(x=x, w=w, bias=bias, q_out=q_out)
-        if q_out is None:
-            q_out = torch.zeros((n, self.opts.n_embd), dtype=torch.float32, device=x.device)
-        qs, _ = self._f32(q_out, "q_out", False, n)
-        self._check(self._L.ni_kv_qkv_append_w(self._h, layer, rp, n, x.data_ptr(), xs, x.shape[1], w.data_ptr(),
+        d_in, c = x.shape[1], self._c
+        xs = _fits(x, n, d_in, self.device)
+        quick = xs is not None
+        if not quick:
+            xs, _ = self._f32(x, "x", False, n, c=d_in)
+        _weights(w, bias, c, d_in, w_format)
+        qs = _fits(q_out, n, c, self.device)
+        if not quick or qs is None or w.get_device() != self.device or (
+                bias is not None and bias.get_device() != self.device):
+            if q_out is not None:
+                self._f32(q_out, "q_out", False, n)
+            self._on_device(x=x, w=w, bias=bias, q_out=q_out)
+            if q_out is None:
+                q_out = torch.zeros((n, c), dtype=torch.float32, device=x.device)
+            qs, _ = self._f32(q_out, "q_out", False, n)
+        self._check(self._L.ni_kv_qkv_append_w(self._h, layer, rp, n, x.data_ptr(), xs, d_in, w.data_ptr(),
                                                W_FORMATS[w_format], None if bias is None else bias.data_ptr(),
                                                q_out.data_ptr(), qs, _stream_ptr(stream)))
         return q_out
@@ -361,17 +428,24 @@ class PagedKv:
 
     def attention(self, q, rows, out=None, layer: int = ALL_LAYERS, split_tokens: int = 0, stream=None):
         """Paged decode attention of each row over keys 0..pos of its sequence."""
-        import torch
-
+        torch = _torch()
         arr, rp, n = _rows(rows)
         layered = layer == ALL_LAYERS
-        qrs, qls = self._f32(q, "q", layered, n)
-        if out is not None:
-            self._f32(out, "out", layered, n)
-        self._on_device(q=q, out=out)
-        if out is None:
-            out = torch.zeros_like(q)
-        ors, ols = self._f32(out, "out", layered, n)
+        if layered:
+            qs = _fits_layers(q, n, self._c, self._n_layer, self.device)
+            os_ = _fits_layers(out, n, self._c, self._n_layer, self.device)
+        else:
+            qs, os_ = _fits(q, n, self._c, self.device), _fits(out, n, self._c, self.device)
+            qs, os_ = None if qs is None else (qs, 0), None if os_ is None else (os_, 0)
+        if qs is None or os_ is None:
+            qs = self._f32(q, "q", layered, n)
+            if out is not None:
+                self._f32(out, "out", layered, n)
+            self._on_device(q=q, out=out)
+            if out is None:
+                out = torch.zeros_like(q)
+            os_ = self._f32(out, "out", layered, n)
+        (qrs, qls), (ors, ols) = qs, os_
         self._check(self._L.ni_paged_decode_attention(self._h, layer, q.data_ptr(), qrs, qls, rp, n, out.data_ptr(),
                                                       ors, ols, split_tokens, _stream_ptr(stream)))
         return out
@@ -380,22 +454,24 @@ class PagedKv:
         """One step over every layer (Batch::step's KV part).  ``work`` lists
         ``(seq, n_new, n_query)``; rows are numbered in work order; q/k/v/out
         are [n_layer, rows, C]."""
-        import torch
-
+        torch = _torch()
         w = _work(work)
-        wp = w.ctypes.data_as(C.POINTER(_abi.ni_work))
+        wp = _pointer(w, _no_work, _abi.ni_work)
         n = _work_rows(w)
-        rs3, ls3 = self._f32(q, "q", True, n)
-        rs, ls = self._f32(k, "k", True, n)
-        rs2, ls2 = self._f32(v, "v", True, n)
-        if not (rs == rs2 == rs3 and ls == ls2 == ls3):
-            raise ValueError("q, k and v must share strides")
-        if out is not None:
-            self._f32(out, "out", True, n)
-        self._on_device(q=q, k=k, v=v, out=out)
-        if out is None:
-            out = torch.zeros_like(q)
-        ors, ols = self._f32(out, "out", True, n)
+        c, n_layer, device = self._c, self._n_layer, self.device
+        s, so = _fits_layers(q, n, c, n_layer, device), _fits_layers(out, n, c, n_layer, device)
+        if s is None or so is None or _fits_layers(k, n, c, n_layer, device) != s \
+                or _fits_layers(v, n, c, n_layer, device) != s:
+            s3, s, s2 = self._f32(q, "q", True, n), self._f32(k, "k", True, n), self._f32(v, "v", True, n)
+            if not s == s2 == s3:
+                raise ValueError("q, k and v must share strides")
+            if out is not None:
+                self._f32(out, "out", True, n)
+            self._on_device(q=q, k=k, v=v, out=out)
+            if out is None:
+                out = torch.zeros_like(q)
+            so = self._f32(out, "out", True, n)
+        (rs, ls), (ors, ols) = s, so
         self._check(self._L.ni_kv_step(self._h, wp, w.shape[0], q.data_ptr(), k.data_ptr(), v.data_ptr(), rs, ls,
                                        out.data_ptr(), ors, ols, split_tokens, _stream_ptr(stream)))
         return out
@@ -406,27 +482,27 @@ class PagedKv:
         does (batch.rs:280-306 encodes once, batch.rs:390-416 dispatches per
         layer); :meth:`step_end` commits it."""
         w = _work(work)
-        self._check(self._L.ni_kv_step_begin(self._h, w.ctypes.data_as(C.POINTER(_abi.ni_work)), w.shape[0],
-                                             split_tokens))
+        self._check(self._L.ni_kv_step_begin(self._h, _pointer(w, _no_work, _abi.ni_work), w.shape[0], split_tokens))
         self._open_rows = _work_rows(w)
 
     def step_layer(self, layer: int, q, k, v, out=None, stream=None):
         """Layer ``layer`` of the open step: its new rows appended and its
         queried rows attended in one launch; q/k/v/out are [rows, C]."""
-        import torch
-
-        n = self._open_rows or 0
-        rs3, _ = self._f32(q, "q", False, n)
-        rs, _ = self._f32(k, "k", False, n)
-        rs2, _ = self._f32(v, "v", False, n)
-        if not rs == rs2 == rs3:
-            raise ValueError("q, k and v must share a row stride")
-        if out is not None:
-            self._f32(out, "out", False, n)
-        self._on_device(q=q, k=k, v=v, out=out)
-        if out is None:
-            out = torch.zeros_like(q)
-        ors, _ = self._f32(out, "out", False, n)
+        torch = _torch()
+        n, c, device = self._open_rows or 0, self._c, self.device
+        rs, ors = _fits(q, n, c, device), _fits(out, n, c, device)
+        if rs is None or ors is None or _fits(k, n, c, device) != rs or _fits(v, n, c, device) != rs:
+            rs3, _ = self._f32(q, "q", False, n)
+            rs, _ = self._f32(k, "k", False, n)
+            rs2, _ = self._f32(v, "v", False, n)
+            if not rs == rs2 == rs3:
+                raise ValueError("q, k and v must share a row stride")
+            if out is not None:
+                self._f32(out, "out", False, n)
+            self._on_device(q=q, k=k, v=v, out=out)
+            if out is None:
+                out = torch.zeros_like(q)
+            ors, _ = self._f32(out, "out", False, n)
         self._check(self._L.ni_kv_step_layer(self._h, layer, q.data_ptr(), k.data_ptr(), v.data_ptr(), rs,
                                              out.data_ptr(), ors, _stream_ptr(stream)))
         return out
@@ -496,29 +572,32 @@ def attention(q, k, v, n_q: int, q_pos0: int, n_head: int, head_dim: int, out=No
     buffer); q holds ``n_q`` rows, k and v at least ``q_pos0 + n_q``, each at
     least ``C = n_head * head_dim`` wide.  Returns ``out`` ([n_q][C] float32,
     allocated if not given).  No scores buffer is needed."""
-    import torch
-
-    c = n_head * head_dim
-    if n_q < 0 or q_pos0 < 0:
-        raise ValueError("n_q and q_pos0 must be >= 0")
-    args = (("q", q, n_q), ("k", k, q_pos0 + n_q), ("v", v, q_pos0 + n_q))
-    for name, t, rows in args:  # layout first, then the device
-        if not isinstance(t, torch.Tensor) or t.dtype != torch.float32 or t.dim() != 2:
-            raise TypeError(f"{name} must be a 2-D float32 tensor")
-        if t.stride(1) != 1:
-            raise ValueError(f"{name} rows must be contiguous")
-        if t.shape[0] < rows or t.shape[1] < c:
-            raise ValueError(f"{name} is {tuple(t.shape)}; needs at least {rows} rows of {c}")
-    for name, t, _ in args:
-        if not t.is_cuda:
-            raise TypeError(f"{name} must be a CUDA tensor")
-        if t.device != q.device:
-            raise ValueError(f"{name} is on {t.device}, q on {q.device}")
-    if out is None:
-        out = torch.empty((n_q, c), dtype=torch.float32, device=q.device)
-    if (not isinstance(out, torch.Tensor) or out.dtype != torch.float32 or out.dim() != 2 or out.stride(1) != 1
-            or out.shape[0] < n_q or out.shape[1] < c or out.device != q.device):
-        raise ValueError(f"out must be a float32 [{n_q}][{c}] tensor on {q.device} with contiguous rows")
+    torch = _torch()
+    c, n_kv = n_head * head_dim, q_pos0 + n_q
+    # The quick form of the checks below, which say what is wrong.
+    device = q.get_device() if type(q) is _Tensor else None
+    if not (n_q >= 0 and q_pos0 >= 0 and _fits_wide(q, n_q, c, device) and _fits_wide(k, n_kv, c, device)
+            and _fits_wide(v, n_kv, c, device) and _fits_wide(out, n_q, c, device)):
+        if n_q < 0 or q_pos0 < 0:
+            raise ValueError("n_q and q_pos0 must be >= 0")
+        args = (("q", q, n_q), ("k", k, q_pos0 + n_q), ("v", v, q_pos0 + n_q))
+        for name, t, rows in args:  # layout first, then the device
+            if not isinstance(t, torch.Tensor) or t.dtype != torch.float32 or t.dim() != 2:
+                raise TypeError(f"{name} must be a 2-D float32 tensor")
+            if t.stride(1) != 1:
+                raise ValueError(f"{name} rows must be contiguous")
+            if t.shape[0] < rows or t.shape[1] < c:
+                raise ValueError(f"{name} is {tuple(t.shape)}; needs at least {rows} rows of {c}")
+        for name, t, _ in args:
+            if not t.is_cuda:
+                raise TypeError(f"{name} must be a CUDA tensor")
+            if t.device != q.device:
+                raise ValueError(f"{name} is on {t.device}, q on {q.device}")
+        if out is None:
+            out = torch.empty((n_q, c), dtype=torch.float32, device=q.device)
+        if (not isinstance(out, torch.Tensor) or out.dtype != torch.float32 or out.dim() != 2 or out.stride(1) != 1
+                or out.shape[0] < n_q or out.shape[1] < c or out.device != q.device):
+            raise ValueError(f"out must be a float32 [{n_q}][{c}] tensor on {q.device} with contiguous rows")
     L = _abi.lib()
     rc = L.ni_attention(out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
                         v.data_ptr(), v.stride(0), n_q, q_pos0, n_head, head_dim, _stream_ptr(stream))
