@@ -1193,11 +1193,27 @@ __device__ __forceinline__ void qkv_store_en(const QkvLaunch& a, const AppendEnt
     }
 }
 
+// What a thread of qkv_kernel loads at once of a W that is not f32: 16 bytes of
+// a row (Q4_0: 8 bytes, half a block) and the block's scale, kElems elements,
+// converted when the chunk goes to LDS.  Four weights at a time (qkv_w4), each
+// with its scale, took as many loads as f32 and kept the conversion between a
+// load and the next: GPT-2, 512 rows f16 27.9 -> 23.0 us, q8_0 28.2 -> 24.3, q4_0
+// 28.1 -> 25.0 (f32 23.1); 128 rows q4_0 12.6 -> 11.9, 1024 rows 52.3 -> 47.0.
+template <int WF>
+struct QkvUnit {
+    static constexpr int kElems = WF == kWF32 ? 4 : WF == kWF16 ? 8 : 16;
+    static constexpr int kPerRow = kQkvChunk / kElems;  // units per chunk of a row
+    u32x4 raw;
+    uint32_t scale;
+};
+
 template <int FB, int INL, int WF>
 __global__ __launch_bounds__(256) void qkv_kernel(const QkvLaunch a, const PlanArg<INL> pa) {
     typedef float f4 __attribute__((ext_vector_type(4)));
     constexpr int TM = kQkvTileRows, TF = 16 * FB, KC = kQkvChunk, KP = kQkvPad;
-    constexpr int XV = TM * KC / 4 / 256, WV = TF * KC / 4 / 256;  // float4 per thread per chunk
+    constexpr int XV = TM * KC / 4 / 256;              // float4 of x per thread per chunk
+    constexpr int UR = QkvUnit<WF>::kPerRow;           // units of W per row and chunk
+    constexpr int NU = (TF * UR + 255) / 256;          // units per thread and chunk
     __shared__ __attribute__((aligned(16))) float xs[TM][KP];
     __shared__ __attribute__((aligned(16))) float ws[TF][KP];
     __shared__ float red[2][FB][4][64];
@@ -1210,7 +1226,9 @@ __global__ __launch_bounds__(256) void qkv_kernel(const QkvLaunch a, const PlanA
     // Staging: float4 u = threadIdx.x + 256 * j of a chunk is row u / (KC/4),
     // column 4 * (u % (KC/4)).  Rows past n_rows repeat the last row; values
     // past d_in (the last, partial chunk) are zeros.
-    float4 xr[XV], wr[WV];
+    constexpr int WV = WF == kWF32 ? TF * KC / 4 / 256 : 1;  // f32 W: float4s, as x
+    float4 xr[XV], wf[WV];
+    QkvUnit<WF> wr[WF == kWF32 ? 1 : NU];
     auto fetch = [&](uint32_t k0) {
 #pragma unroll
         for (int j = 0; j < XV; j++) {
@@ -1219,14 +1237,78 @@ __global__ __launch_bounds__(256) void qkv_kernel(const QkvLaunch a, const PlanA
             xr[j] = k0 + col < a.d_in ? *reinterpret_cast<const float4*>(a.x + (int64_t)r * a.x_row_stride + k0 + col)
                                       : float4{0.f, 0.f, 0.f, 0.f};
         }
+        if constexpr (WF == kWF32) {
 #pragma unroll
-        for (int j = 0; j < WV; j++) {
-            const uint32_t u = threadIdx.x + 256 * j, row = u / (KC / 4), col = 4 * (u % (KC / 4));
-            if (k0 + col < a.d_in) {
-                const qkv_f4 v = qkv_w4<WF>(a, n0 + row, k0 + col);
-                wr[j] = float4{v[0], v[1], v[2], v[3]};
-            } else {
-                wr[j] = float4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < WV; j++) {
+                const uint32_t u = threadIdx.x + 256 * j, row = u / (KC / 4), col = 4 * (u % (KC / 4));
+                if (k0 + col < a.d_in) {
+                    const qkv_f4 v = qkv_w4<WF>(a, n0 + row, k0 + col);
+                    wf[j] = float4{v[0], v[1], v[2], v[3]};
+                } else {
+                    wf[j] = float4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NU; j++) {
+                const uint32_t u = threadIdx.x + 256 * j, row = u / UR, c = u % UR;
+                if (TF * UR % 256 != 0 && row >= (uint32_t)TF) break;
+                // (Q4_0: unit 2b + h of a row is bytes 8h .. 8h+7 of block b, the
+                // low nibbles elements 8h .., the high ones 16 + 8h ..)
+                const uint32_t col = k0 + (WF == kWQ4 ? c / 2 * 32 : c * QkvUnit<WF>::kElems);
+                const uint8_t* const wb = static_cast<const uint8_t*>(a.w);
+                const uint64_t e = (uint64_t)(n0 + row) * a.d_in + col, n = (uint64_t)a.n_feat * a.d_in;
+                wr[j].raw = u32x4{0u, 0u, 0u, 0u};
+                wr[j].scale = 0u;
+                if (col >= a.d_in) continue;
+                if constexpr (WF == kWF16) {
+                    wr[j].raw = *reinterpret_cast<const u32x4*>(wb + 2 * e);
+                } else {
+                    if constexpr (WF == kWQ8) {
+                        wr[j].raw = *reinterpret_cast<const u32x4*>(wb + e);
+                    } else {
+                        const uint2 q = *reinterpret_cast<const uint2*>(wb + e / 2 + 8 * (c % 2));
+                        wr[j].raw.x = q.x;
+                        wr[j].raw.y = q.y;
+                    }
+                    wr[j].scale = reinterpret_cast<const uint16_t*>(wb + (WF == kWQ8 ? n : n / 2))[e / 32];
+                }
+            }
+        }
+    };
+    // W's rows of the chunk: a unit's elements as f32 (exactly, as qkv_w4).
+    auto stage_w = [&]() {
+        if constexpr (WF == kWF32) {
+#pragma unroll
+            for (int j = 0; j < WV; j++) {
+                const uint32_t u = threadIdx.x + 256 * j;
+                *reinterpret_cast<float4*>(&ws[u / (KC / 4)][4 * (u % (KC / 4))]) = wf[j];
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NU; j++) {
+                const uint32_t u = threadIdx.x + 256 * j, row = u / UR, c = u % UR;
+                if (TF * UR % 256 != 0 && row >= (uint32_t)TF) break;
+                f4* const dst = reinterpret_cast<f4*>(&ws[row][0]);
+                if constexpr (WF == kWF16) {
+                    const half8_t hv = __builtin_bit_cast(half8_t, wr[j].raw);
+                    dst[2 * c] = f4{(float)hv[0], (float)hv[1], (float)hv[2], (float)hv[3]};
+                    dst[2 * c + 1] = f4{(float)hv[4], (float)hv[5], (float)hv[6], (float)hv[7]};
+                } else {
+                    const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)wr[j].scale);
+#pragma unroll
+                    for (int w = 0; w < 4; w++) {
+                        if constexpr (WF == kWQ8) {
+                            const uint32_t q = wr[j].raw[w];
+                            dst[4 * c + w] = f4{i8f(q, 0) * d, i8f(q, 1) * d, i8f(q, 2) * d, i8f(q, 3) * d};
+                        } else {
+                            const uint32_t q = wr[j].raw[w & 1] >> (w >= 2 ? 4 : 0);
+                            dst[c / 2 * 8 + (w >= 2 ? 4 : 0) + 2 * (c % 2) + (w & 1)] =
+                                f4{(float)((int)(q & 15u) - 8) * d, (float)((int)((q >> 8) & 15u) - 8) * d,
+                                   (float)((int)((q >> 16) & 15u) - 8) * d, (float)((int)((q >> 24) & 15u) - 8) * d};
+                        }
+                    }
+                }
             }
         }
     };
@@ -1244,11 +1326,7 @@ __global__ __launch_bounds__(256) void qkv_kernel(const QkvLaunch a, const PlanA
             const uint32_t u = threadIdx.x + 256 * j;
             *reinterpret_cast<float4*>(&xs[u / (KC / 4)][4 * (u % (KC / 4))]) = xr[j];
         }
-#pragma unroll
-        for (int j = 0; j < WV; j++) {
-            const uint32_t u = threadIdx.x + 256 * j;
-            *reinterpret_cast<float4*>(&ws[u / (KC / 4)][4 * (u % (KC / 4))]) = wr[j];
-        }
+        stage_w();
         __syncthreads();
         if (k0 + KC < a.d_in) fetch(k0 + KC);
         // This wave's half of the chunk: slices of 16, slice sl of the half
