@@ -423,6 +423,54 @@ void balance_prefill_units(Plan& P, uint32_t n_lay, uint32_t n_head, uint64_t C,
     deal_units(cost, lh, C, R, rem, P.porder);
 }
 
+// Whether a launch of prompt chunks runs faster as groups of one matrix tile
+// on the group kernel (kWideWaves waves per workgroup share a group's pages at
+// head_dim 64, kWaves at 128) than as prefill groups of 64 rows: those read each
+// key once per 64 rows, but put a short launch on few CUs, whose chain of key
+// tiles it then waits for.  Both sides in us per launch, measured on MI355X with
+// 12 heads x 64 (32 x 128), the larger of the longest item's chain and the
+// launch's share of work per CU:
+// * prefill groups: 3 (Q8 3.4), plus 0.55 per 32-key tile of the longest
+//   (head_dim 128: per 16 keys; Q8: 1.15), or 0.39 (Q8 0.57) per tile a CU
+//   receives;
+// * tile groups: 4.6, plus 0.75 per round of the waves over the longest's pages
+//   (head_dim 128: 1.08), or 0.6 per group and 0.115 per page (0.3) a CU
+//   receives.
+// One layer, one prompt, prefill / tile groups: 64 rows 4.3 / 4.7, 320 rows 8.4 /
+// 6.3, 509 rows 12.0 / 8.7, 64 rows after 300 9.3 / 6.8, after 2000 36.9 / 16.2; 2 x
+// 256 rows 7.9 / 7.7, 5 x 256 8.5 / 9.8; Q8 100 rows 7.2 / 5.3, 509 rows 19.3 /
+// 9.6; head_dim 128 256 rows 12.4 / 10.6, 500 rows 21 / 23; 12 layers 100 rows 5.7
+// / 7.6, Q8 500 rows after 300 54 / 74.
+bool small_groups(ni_kv* kv, uint32_t n_lay) {
+    const Plan& P = kv->plan;
+    const auto& qr = kv->qrows;
+    // (a fused or prompt-chunk plan's chunks must run in the prefill launch;
+    // ni_kv_step_noalloc keeps the sizes of step it takes)
+    if (P.fused || P.seq_prefill || kv->no_alloc) return false;
+    const bool q8 = is_q8(kv->o), d64 = kv->o.head_dim == 64;
+    uint64_t pages = 0, groups = 0, tiles = 0, max_pages = 0;  // of tile groups; 32-key tiles of prefill groups
+    for (size_t i = 0; i < qr.size();) {
+        size_t e = i + 1;
+        while (e < qr.size() && qr[e].seq == qr[i].seq && qr[e].row == qr[e - 1].row + 1 && qr[e].pos == qr[e - 1].pos + 1)
+            e++;
+        if (e - i <= kMfmaTile) return false;  // not a launch of prompt chunks only
+        const uint32_t end = qr[e - 1].pos + 1;
+        for (uint32_t p = qr[i].pos; p < end; p += kMfmaTile, groups++)
+            pages += (std::min(p + kMfmaTile, end) + kPage - 1) / kPage;
+        for (uint32_t p = qr[i].pos; p < end; p += kPrefillRows) tiles += (std::min(p + kPrefillRows, end) + 31) / 32;
+        max_pages = std::max<uint64_t>(max_pages, (end + kPage - 1) / kPage);
+        i = e;
+    }
+    const double per_cu = (double)n_lay * kv->o.n_head / device_cus();
+    const double per_tile = q8 ? 1.15 : 0.55, tile_load = q8 ? 0.57 : 0.39;
+    const double chain64 = per_tile * (d64 ? (max_pages + 1) / 2 : max_pages);
+    const double us64 = (q8 ? 3.4 : 3.0) + std::max(chain64, tile_load * (d64 ? 1 : 2) * per_cu * tiles);
+    const uint64_t waves = d64 ? kWideWaves : 4;
+    const double us16 = 4.6 + std::max((d64 ? 0.75 : 1.08) * ((max_pages + waves - 1) / waves),
+                                       per_cu * (0.6 * groups + (d64 ? 0.115 : 0.3) * pages));
+    return us16 < us64;
+}
+
 // Attention part of a plan: group consecutive query rows of one sequence at
 // consecutive positions, split each group's keys into partitions, sort the
 // items longest first.
@@ -440,7 +488,8 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
     // Runs longer than one matrix tile form prefill groups (f16 pools, and Q8
     // pools at head_dim 64).
     const bool prefill = !is_q8(kv->o) || kv->o.head_dim == 64;
-    const uint32_t max_group = prefill ? kPrefillRows : max_group_rows(kv);
+    const uint32_t max_group =
+        prefill && (split_tokens || !small_groups(kv, n_lay)) ? kPrefillRows : max_group_rows(kv);
     for (const QRow& r : qr) {
         if (!groups.empty()) {
             Group& g = groups.back();
@@ -451,6 +500,15 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
         }
         groups.push_back({r.seq, r.row, r.pos, 1, r.new_begin, r.new_end, r.app_first, r.pre});
     }
+    // A run's last group joins the others' prefill launch however short it is
+    // (a group-kernel launch of its own after theirs: 200 rows from empty, one
+    // layer 11.3 against 7.3 us; 12 layers 15.5 against 9.2).
+    if (max_group == kPrefillRows)
+        for (size_t i = 1; i < groups.size(); i++) {
+            Group& g = groups[i];
+            const Group& b = groups[i - 1];
+            if (b.nq == kPrefillRows && b.seq == g.seq && b.row0 + b.nq == g.row0 && b.pos0 + b.nq == g.pos0) g.pre = 1;
+        }
     // Partition size: the caller's, or (0) automatic.  Splitting costs a
     // merge launch (~5-7 us) and the partials' round trip, so it pays only
     // when the unsplit items cannot keep the GPU busy: 256 CUs hold 1024
