@@ -3515,11 +3515,24 @@ hipError_t launch_qkv_t(const QkvLaunch& a, const void* ip, uint32_t ib, hipStre
             });
         }
     }
-    const dim3 grid(row_tiles, a.n_feat / kQkvTileFeat);
+    // Otherwise 32-feature tiles (x read by half as many workgroups, 38 KB of
+    // LDS, 4 per CU) where the CU with the most of them gets no more 16-feature
+    // blocks than with 16-feature tiles: us per layer of GPT-2, 16 / 32 wide, 440
+    // rows f32 23.9 / 21.3, f16 24.0 / 21.0, q4_0 24.9 / 22.3; 640 rows f32 31.5 /
+    // 29.7, q4_0 34.9 / 32.1.  One block more loses where it starts a round
+    // (480 rows f32 24.8 / 26.7), and below 8 blocks there are too few
+    // workgroups to hide a chunk's loads (224 rows q8_0 13.4 / 13.8).
+    const uint64_t cus = device_cus();
+    auto blocks = [&](uint64_t fb) { return ((uint64_t)row_tiles * (a.n_feat / (16 * fb)) + cus - 1) / cus * fb; };
+    const bool pair = a.n_feat % 32 == 0 && blocks(1) >= 8 && blocks(2) <= blocks(1);
     return with_plan(a, ip, ib, [&](auto pa) {
         constexpr int INL = sizeof(pa.b) > 4 ? (int)sizeof(pa.b) : 0;
-        hipExtLaunchKernelGGL(qkv_kernel<kQkvTileFeat / 16, INL, WF>, grid, dim3(256), 0, s, t.start, t.stop, 0, a,
-                              pa);
+        if (pair)
+            hipExtLaunchKernelGGL(qkv_kernel<2, INL, WF>, dim3(row_tiles, a.n_feat / 32), dim3(256), 0, s, t.start,
+                                  t.stop, 0, a, pa);
+        else
+            hipExtLaunchKernelGGL(qkv_kernel<kQkvTileFeat / 16, INL, WF>, dim3(row_tiles, a.n_feat / kQkvTileFeat),
+                                  dim3(256), 0, s, t.start, t.stop, 0, a, pa);
         return hipGetLastError();
     });
 }
