@@ -500,15 +500,6 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
         }
         groups.push_back({r.seq, r.row, r.pos, 1, r.new_begin, r.new_end, r.app_first, r.pre});
     }
-    // A run's last group joins the others' prefill launch however short it is
-    // (a group-kernel launch of its own after theirs: 200 rows from empty, one
-    // layer 11.3 against 7.3 us; 12 layers 15.5 against 9.2).
-    if (max_group == kPrefillRows)
-        for (size_t i = 1; i < groups.size(); i++) {
-            Group& g = groups[i];
-            const Group& b = groups[i - 1];
-            if (b.nq == kPrefillRows && b.seq == g.seq && b.row0 + b.nq == g.row0 && b.pos0 + b.nq == g.pos0) g.pre = 1;
-        }
     // Partition size: the caller's, or (0) automatic.  Splitting costs a
     // merge launch (~5-7 us) and the partials' round trip, so it pays only
     // when the unsplit items cannot keep the GPU busy: 256 CUs hold 1024
