@@ -449,11 +449,19 @@ bool small_groups(ni_kv* kv, uint32_t n_lay) {
     if (P.fused || P.seq_prefill || kv->no_alloc) return false;
     const bool q8 = is_q8(kv->o), d64 = kv->o.head_dim == 64;
     uint64_t pages = 0, groups = 0, tiles = 0, max_pages = 0;  // of tile groups; 32-key tiles of prefill groups
+    // After prefill groups, the runs' last 1..16 rows are a launch of their
+    // own: on the row kernel, q and the weights in f32, if each is one row
+    // (which as part of a tile group would be f16 pairs), else on the group
+    // kernel.
+    bool last_row = false, last_group = false;
     for (size_t i = 0; i < qr.size();) {
         size_t e = i + 1;
         while (e < qr.size() && qr[e].seq == qr[i].seq && qr[e].row == qr[e - 1].row + 1 && qr[e].pos == qr[e - 1].pos + 1)
             e++;
         if (e - i <= kMfmaTile) return false;  // not a launch of prompt chunks only
+        const size_t last = (e - i) % kPrefillRows;
+        last_row |= last == 1;
+        last_group |= last > 1 && last <= kMfmaTile;
         const uint32_t end = qr[e - 1].pos + 1;
         for (uint32_t p = qr[i].pos; p < end; p += kMfmaTile, groups++)
             pages += (std::min(p + kMfmaTile, end) + kPage - 1) / kPage;
@@ -461,6 +469,7 @@ bool small_groups(ni_kv* kv, uint32_t n_lay) {
         max_pages = std::max<uint64_t>(max_pages, (end + kPage - 1) / kPage);
         i = e;
     }
+    if (last_row && !last_group) return false;
     const double per_cu = (double)n_lay * kv->o.n_head / device_cus();
     const double per_tile = q8 ? 1.15 : 0.55, tile_load = q8 ? 0.57 : 0.39;
     const double chain64 = per_tile * (d64 ? (max_pages + 1) / 2 : max_pages);

@@ -103,7 +103,8 @@ def _rel(got, want):
 
 
 @pytest.mark.parametrize("head_dim", [64, 128])
-@pytest.mark.parametrize("n_layer,ctx,rows", [(12, 0, 65), (12, 0, 129), (12, 150, 193)], ids=str)
+@pytest.mark.parametrize("n_layer,ctx,rows", [(12, 0, 65), (12, 0, 129), (12, 150, 193), (1, 0, 65), (1, 0, 513),
+                                              (1, 300, 129)], ids=str)
 def test_a_single_last_row_is_f32(gpu, n_layer, ctx, rows, head_dim):
     """The row a prompt's first token comes from.  Its query scaled past f16's
     range (2^19 |q| log2(e) / sqrt(head_dim): past 65504 an f16 pair is
