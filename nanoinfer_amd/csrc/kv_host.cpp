@@ -444,9 +444,8 @@ void balance_prefill_units(Plan& P, uint32_t n_lay, uint32_t n_head, uint64_t C,
 bool small_groups(ni_kv* kv, uint32_t n_lay) {
     const Plan& P = kv->plan;
     const auto& qr = kv->qrows;
-    // (a fused or prompt-chunk plan's chunks must run in the prefill launch;
-    // ni_kv_step_noalloc keeps the sizes of step it takes)
-    if (P.fused || P.seq_prefill || kv->no_alloc) return false;
+    // (a fused or prompt-chunk plan's chunks must run in the prefill launch)
+    if (P.fused || P.seq_prefill) return false;
     const bool q8 = is_q8(kv->o), d64 = kv->o.head_dim == 64;
     uint64_t pages = 0, groups = 0, tiles = 0, max_pages = 0;  // of tile groups; 32-key tiles of prefill groups
     // After prefill groups, the runs' last 1..16 rows are a launch of their
@@ -480,127 +479,192 @@ bool small_groups(ni_kv* kv, uint32_t n_lay) {
     return us16 < us64;
 }
 
-// Attention part of a plan: group consecutive query rows of one sequence at
-// consecutive positions, split each group's keys into partitions, sort the
-// items longest first.
-int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
-    Plan& P = kv->plan;
-    const auto& qr = kv->qrows;
-    if (qr.empty()) return NI_OK;
-    struct Group {
-        uint32_t seq, row0, pos0, nq;
-        uint32_t new_begin, new_end, app_first;
-        uint32_t pre;  // runs in the prefill launch whatever its size
-    };
+// Query rows that share a pass over their sequence's keys.
+struct Group {
+    uint32_t seq, row0, pos0, nq;
+    uint32_t new_begin, new_end, app_first;
+    uint32_t pre;  // runs in the prefill launch whatever its size
+    uint32_t keys() const { return pos0 + nq; }
+    bool prefill() const { return pre || nq > kMfmaTile; }
+};
+
+// Groups of at most max_rows consecutive rows of one sequence at consecutive
+// positions.
+std::vector<Group> form_groups(const std::vector<QRow>& qr, uint32_t max_rows) {
     std::vector<Group> groups;
     groups.reserve(qr.size());
-    // Runs longer than one matrix tile form prefill groups (f16 pools, and Q8
-    // pools at head_dim 64).
-    const bool prefill = !is_q8(kv->o) || kv->o.head_dim == 64;
-    const uint32_t max_group =
-        prefill && (split_tokens || !small_groups(kv, n_lay)) ? kPrefillRows : max_group_rows(kv);
     for (const QRow& r : qr) {
         if (!groups.empty()) {
             Group& g = groups.back();
-            if (g.seq == r.seq && g.row0 + g.nq == r.row && g.pos0 + g.nq == r.pos && g.nq < max_group) {
+            if (g.seq == r.seq && g.row0 + g.nq == r.row && g.pos0 + g.nq == r.pos && g.nq < max_rows) {
                 g.nq++;
                 continue;
             }
         }
         groups.push_back({r.seq, r.row, r.pos, 1, r.new_begin, r.new_end, r.app_first, r.pre});
     }
-    // Partition size: the caller's, or (0) automatic.  Splitting costs a
-    // merge launch (~5-7 us) and the partials' round trip, so it pays only
-    // when the unsplit items cannot keep the GPU busy: 256 CUs hold 1024
-    // workgroups at once, and with >= 2048 of them, sorted longest first,
-    // the tail is short -- only items longer than kLongItem keys are split
-    // then.  Below that, the largest of 1024/512/256/128 tokens that yields
-    // >= 2048 workgroups.
-    // At head_dim 64, launches of single rows or of groups within one matrix
-    // tile below that are not split either: several waves of one workgroup
-    // share each item's pages and merge in LDS, no partials, no merge launch
-    // (us per launch, split and merged against one workgroup per item):
-    // * single rows: kWideWaves waves (Q8: kWideWavesQ8), kSoloWaves while
-    //   every unit has a CU of its own and the items are long enough to keep
-    //   16 waves busy, kWaves up to kNarrowKeys keys, where waves of 2 pages
-    //   cover an item at once.  12 layers x 12 heads: 1 sequence of 150 keys
-    //   7.1 / 3.9, 300 7.9 / 5.2, 517 9.2 / 6.6, 1000 11.5 / 9.1, 3000 24.3 /
-    //   20.5, 3 of 1000 24.3 / 19.0; Q8 517 9.9 / 7.0, 3 of 1000 21.0 / 13.2.
-    // * groups: kWideWaves waves below kWideMinUnits units (12 layers, 5 rows of
-    //   300 keys 8.2 / 5.8, 1000 13.7 / 10.1), from there on, where two such
-    //   workgroups no longer fit each CU, kWaves (4 x U[64,1000] 23.2 -> 19.5,
-    //   13 41.9 -> 37.0).
-    // Below kWholeMinUnits units that holds up to kShortItem keys only: longer
-    // items fill the GPU faster in partitions (one layer of 12 heads: 1
-    // sequence of 2000 keys 8.1 / 12.5, 4 of 2000 11.4 / 13.4, 16 of 2000 24.1 /
-    // 18.8).
-    // Prefill groups (more rows than one matrix tile, in a launch of their
-    // own) are split automatically only past kLongItem keys: each of their
-    // workgroups already carries 64 queries, and splitting them to fill the
-    // GPU cost more than it gained (prompt steps, every row queried, no split
-    // against the fill choice: one launch per layer 16 x 512 rows 611 against
-    // 753 us, 4 x 512 286 against 436, 1 x 512 254 against 305; all layers 1 x
-    // 512 45 against 67 us, 4 x 512 146 against 167, 2 x 512 and 8 x 256 the
-    // same).
-    constexpr uint32_t kLongItem = 4096;
-    uint32_t part = split_tokens, pre_part = split_tokens;
-    if (part == 0) {
-        constexpr uint64_t kFillWorkgroups = 2048;
-        constexpr uint64_t kWideMinUnits = 512;
-        constexpr uint64_t kWholeMinUnits = 96;
-        constexpr uint32_t kNarrowKeys = 128, kSoloKeys = 384, kSoloKeysQ8 = 640;
-        static const uint32_t kChoices[] = {1024, 512, 256, 128};
-        pre_part = kLongItem;
-        const uint64_t per_unit = (uint64_t)n_lay * kv->o.n_head;
-        const uint64_t units = (uint64_t)groups.size() * per_unit;
-        constexpr uint32_t kShortItem = 1280;  // keys (a 1024-token context and its new rows)
-        const uint32_t whole_keys = units >= kWholeMinUnits ? kLongItem : kShortItem;
-        bool single = true, tiles = true;  // every group one row; every group within one matrix tile
-        uint32_t max_keys = 0;
-        for (const Group& g : groups) {
-            single &= g.nq == 1;
-            tiles &= g.nq <= kMfmaTile && !g.pre;
-            max_keys = std::max(max_keys, g.pos0 + g.nq);
-        }
-        if (units >= kFillWorkgroups) {
-            part = kLongItem;
-        } else if (tiles && kv->o.head_dim == 64 &&
-                   (units >= (single ? kWideMinUnits : kWideMinUnits / 2) || max_keys <= whole_keys)) {
-            part = kLongItem;
-            const uint32_t solo_keys = is_q8(kv->o) ? kSoloKeysQ8 : kSoloKeys;
-            if (!single)
-                P.wide = units < kWideMinUnits ? 1u : 0u;
-            else if (units >= kWideMinUnits || max_keys > kNarrowKeys)
-                P.wide = units <= device_cus() && max_keys > solo_keys ? 2u : 1u;
-        } else if (n_lay == 1 && max_keys <= kShortItem) {
-            // One layer per launch and no item past kShortItem keys: the
-            // merge launch a split needs costs more than the fill it buys
-            // (decode rows of 4..32 sequences with contexts U[64,1024]: 213-240
-            // against 251-284 us per step of 12 such launches; 8 x 1024 keys
-            // 208 against 246; from 2048 keys the split wins, 4 x 2048 242
-            // against 285, 4 x 4096 246 against 524, and 16 x U[1024,2048]
-            // 262 against 273).
-            part = kLongItem;
-        } else {
-            part = kChoices[3];
-            for (uint32_t c : kChoices) {
-                uint64_t items = 0;
-                for (const Group& g : groups) items += ((uint64_t)g.pos0 + g.nq + c - 1) / c;
-                if (items * per_unit >= kFillWorkgroups) {
-                    part = c;
-                    break;
-                }
+    return groups;
+}
+
+// How a launch cuts its groups: keys per partition, of groups of up to one
+// matrix tile and of prefill groups, and the former's workgroups
+// (AttnLaunch::wide).
+struct Cut {
+    uint32_t part, pre_part, wide;
+    uint32_t n_parts(const Group& g) const {
+        const uint32_t p = g.prefill() ? pre_part : part;
+        return (g.keys() + p - 1) / p;
+    }
+};
+
+// The automatic cut (split_tokens 0).  Splitting costs a merge launch (~5-7
+// us) and the partials' round trip, so it pays only when the unsplit items
+// cannot keep the GPU busy: 256 CUs hold 1024 workgroups at once, and with >=
+// 2048 of them, sorted longest first, the tail is short -- only items longer
+// than kLongItem keys are split then.  Below that, the largest of
+// 1024/512/256/128 tokens that yields >= 2048 workgroups.
+// At head_dim 64, launches of single rows or of groups within one matrix
+// tile below that are not split either: several waves of one workgroup
+// share each item's pages and merge in LDS, no partials, no merge launch
+// (us per launch, split and merged against one workgroup per item):
+// * single rows: kWideWaves waves (Q8: kWideWavesQ8), kSoloWaves while
+//   every unit has a CU of its own and the items are long enough to keep
+//   16 waves busy, kWaves up to kNarrowKeys keys, where waves of 2 pages
+//   cover an item at once.  12 layers x 12 heads: 1 sequence of 150 keys
+//   7.1 / 3.9, 300 7.9 / 5.2, 517 9.2 / 6.6, 1000 11.5 / 9.1, 3000 24.3 /
+//   20.5, 3 of 1000 24.3 / 19.0; Q8 517 9.9 / 7.0, 3 of 1000 21.0 / 13.2.
+// * groups: kWideWaves waves below kWideMinUnits units (12 layers, 5 rows of
+//   300 keys 8.2 / 5.8, 1000 13.7 / 10.1), from there on, where two such
+//   workgroups no longer fit each CU, kWaves (4 x U[64,1000] 23.2 -> 19.5,
+//   13 41.9 -> 37.0).
+// Below kWholeMinUnits units that holds up to kShortItem keys only: longer
+// items fill the GPU faster in partitions (one layer of 12 heads: 1
+// sequence of 2000 keys 8.1 / 12.5, 4 of 2000 11.4 / 13.4, 16 of 2000 24.1 /
+// 18.8).
+// Prefill groups (more rows than one matrix tile, in a launch of their
+// own) are split automatically only past kLongItem keys: each of their
+// workgroups already carries 64 queries, and splitting them to fill the
+// GPU cost more than it gained (prompt steps, every row queried, no split
+// against the fill choice: one launch per layer 16 x 512 rows 611 against
+// 753 us, 4 x 512 286 against 436, 1 x 512 254 against 305; all layers 1 x
+// 512 45 against 67 us, 4 x 512 146 against 167, 2 x 512 and 8 x 256 the
+// same).
+constexpr uint32_t kLongItem = 4096;
+Cut auto_cut(const ni_kv* kv, const std::vector<Group>& groups, uint32_t n_lay) {
+    constexpr uint64_t kFillWorkgroups = 2048;
+    constexpr uint64_t kWideMinUnits = 512;
+    constexpr uint64_t kWholeMinUnits = 96;
+    constexpr uint32_t kNarrowKeys = 128, kSoloKeys = 384, kSoloKeysQ8 = 640;
+    static const uint32_t kChoices[] = {1024, 512, 256, 128};
+    Cut cut{kLongItem, kLongItem, 0};
+    const uint64_t per_unit = (uint64_t)n_lay * kv->o.n_head;
+    const uint64_t units = (uint64_t)groups.size() * per_unit;
+    constexpr uint32_t kShortItem = 1280;  // keys (a 1024-token context and its new rows)
+    const uint32_t whole_keys = units >= kWholeMinUnits ? kLongItem : kShortItem;
+    bool single = true, tiles = true;  // every group one row; every group within one matrix tile
+    uint32_t max_keys = 0;
+    for (const Group& g : groups) {
+        single &= g.nq == 1;
+        tiles &= g.nq <= kMfmaTile && !g.pre;
+        max_keys = std::max(max_keys, g.pos0 + g.nq);
+    }
+    if (units >= kFillWorkgroups) {
+        cut.part = kLongItem;
+    } else if (tiles && kv->o.head_dim == 64 &&
+               (units >= (single ? kWideMinUnits : kWideMinUnits / 2) || max_keys <= whole_keys)) {
+        cut.part = kLongItem;
+        const uint32_t solo_keys = is_q8(kv->o) ? kSoloKeysQ8 : kSoloKeys;
+        if (!single)
+            cut.wide = units < kWideMinUnits ? 1u : 0u;
+        else if (units >= kWideMinUnits || max_keys > kNarrowKeys)
+            cut.wide = units <= device_cus() && max_keys > solo_keys ? 2u : 1u;
+    } else if (n_lay == 1 && max_keys <= kShortItem) {
+        // One layer per launch and no item past kShortItem keys: the
+        // merge launch a split needs costs more than the fill it buys
+        // (decode rows of 4..32 sequences with contexts U[64,1024]: 213-240
+        // against 251-284 us per step of 12 such launches; 8 x 1024 keys
+        // 208 against 246; from 2048 keys the split wins, 4 x 2048 242
+        // against 285, 4 x 4096 246 against 524, and 16 x U[1024,2048]
+        // 262 against 273).
+        cut.part = kLongItem;
+    } else {
+        cut.part = kChoices[3];
+        for (uint32_t c : kChoices) {
+            uint64_t items = 0;
+            for (const Group& g : groups) items += ((uint64_t)g.pos0 + g.nq + c - 1) / c;
+            if (items * per_unit >= kFillWorkgroups) {
+                cut.part = c;
+                break;
             }
         }
-    } else if (part % kPage != 0 || part < kMinSplit) {
+    }
+    return cut;
+}
+
+// Whether ni_kv_step_noalloc takes a launch cut this way (its plan inline, its
+// partials in the scratch array).  ni_kv_step asks too, so that both run the
+// same groups.
+bool noalloc_takes(const ni_kv* kv, const std::vector<Group>& groups, const Cut& cut, uint32_t n_lay, size_t n_table) {
+    const uint64_t lh = (uint64_t)n_lay * kv->o.n_head;
+    size_t items[2] = {0, 0}, merges[2] = {0, 0}, slots[2] = {0, 0};  // [prefill launch]
+    uint32_t nq_tile = 1;
+    for (const Group& g : groups) {
+        const bool pre = g.prefill();
+        const uint32_t n = cut.n_parts(g);
+        items[pre] += n;
+        if (n > 1) {
+            merges[pre]++;
+            slots[pre] += n;
+        }
+        if (!pre && g.nq > 1) nq_tile = kMfmaTile;
+    }
+    size_t bytes = 0;
+    auto add = [&](size_t n, size_t size) { bytes = align_up(bytes + n * size, kAlign); };
+    add(kv->plan.app.size(), sizeof(AppendEntry));
+    add(kv->plan.orphans.size(), sizeof(AppendEntry));
+    for (int p = 0; p < 2; p++) {
+        add(items[p], sizeof(AttnItem));
+        add(merges[p], sizeof(MergeItem));
+    }
+    add(n_table, sizeof(uint32_t));
+    if (cut.wide) add(items[0] * lh, sizeof(uint16_t));  // the order of its units
+    const size_t partials = (slots[0] * nq_tile + slots[1] * kPrefillRows) * lh * (kv->o.head_dim + 2) * sizeof(float);
+    return bytes <= kInlinePlanBytes && partials <= kScratchBytes;
+}
+
+// Attention part of a plan: group the query rows, cut each group's keys into
+// partitions, sort the items longest first.
+int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
+    Plan& P = kv->plan;
+    const auto& qr = kv->qrows;
+    if (qr.empty()) return NI_OK;
+    if (split_tokens && (split_tokens % kPage != 0 || split_tokens < kMinSplit))
         return kv->fail(NI_ERR_BAD_ARG, "split_tokens %u must be 0 or a multiple of 16 that is >= %u", split_tokens,
                         kMinSplit);
-    }
+    // Runs longer than one matrix tile form prefill groups (f16 pools, and Q8
+    // pools at head_dim 64).
+    const bool prefill = !is_q8(kv->o) || kv->o.head_dim == 64;
+    std::vector<Group> groups = form_groups(qr, prefill ? kPrefillRows : max_group_rows(kv));
     // Page lists: one segment per sequence, long enough for its last query.
+    size_t n_table = 0;
     for (const Group& g : groups) {
-        const uint32_t need = (g.pos0 + g.nq + kPage - 1) / kPage;
+        const uint32_t need = (g.keys() + kPage - 1) / kPage;
+        n_table += need > kv->seq_need[g.seq] ? need - kv->seq_need[g.seq] : 0;
         kv->seq_need[g.seq] = std::max(kv->seq_need[g.seq], need);
     }
+    Cut cut{split_tokens, split_tokens, 0};
+    if (split_tokens == 0) {
+        cut = auto_cut(kv, groups, n_lay);
+        if (prefill && small_groups(kv, n_lay)) {
+            std::vector<Group> tiles = form_groups(qr, max_group_rows(kv));
+            const Cut c = auto_cut(kv, tiles, n_lay);
+            if (noalloc_takes(kv, tiles, c, n_lay, n_table) || !noalloc_takes(kv, groups, cut, n_lay, n_table)) {
+                groups.swap(tiles);
+                cut = c;
+            }
+        }
+    }
+    P.wide = cut.wide;
     for (const Group& g : groups) {
         if (kv->seq_tab[g.seq] >= 0) continue;
         kv->seq_tab[g.seq] = (int64_t)P.table.size();
@@ -630,7 +694,7 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
                 P.napp_total += it.napp;
             }
         }
-        (g.pre || g.nq > kMfmaTile ? P.pitems : P.items).push_back(it);
+        (g.prefill() ? P.pitems : P.items).push_back(it);
     };
     // Per sequence (page-list offset): its appended rows, for prefill
     // workgroups that append them (P.seq_prefill).
@@ -639,16 +703,16 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
     };
     std::vector<SeqRows> app_of;  // by table offset
     for (const Group& g : groups) {
-        const bool pre = g.pre || g.nq > kMfmaTile;
+        const bool pre = g.prefill();
         if (P.seq_prefill) {
             const uint32_t tab = (uint32_t)kv->seq_tab[g.seq];
             if (app_of.size() <= tab) app_of.resize(tab + 1, {0u, 0u, 0u});
             app_of[tab] = {g.app_first, g.new_begin, g.new_end};
         }
         if (!pre) max_nq = std::max(max_nq, g.nq);
-        const uint32_t L = g.pos0 + g.nq;
-        const uint32_t gpart = pre ? pre_part : part;
-        const uint32_t n_parts = (L + gpart - 1) / gpart;
+        const uint32_t L = g.keys();
+        const uint32_t gpart = pre ? cut.pre_part : cut.part;
+        const uint32_t n_parts = cut.n_parts(g);
         const uint32_t tab = (uint32_t)kv->seq_tab[g.seq];
         if (n_parts <= 1) {
             item(g, tab, 0, L, kNoSlot);

@@ -151,6 +151,49 @@ def test_noalloc_q8_prompt_chunks_appended_by_the_prefill_launch(gpu):
     b.close()
 
 
+# (n_layer, head_dim, contexts, rows): prompt chunks with the automatic cut.  The last is 27 prompts of 64 rows, one
+# after a long context: as 16-row groups its plan would be past 32 KB, as 64-row groups it is not.
+PROMPTS = [(1, 64, [0], [100]), (1, 64, [0], [509]), (12, 64, [0], [64]), (12, 64, [300], [40]), (2, 64, [0, 70], [200, 90]),
+           (12, 64, [0], [200]), (1, 128, [0], [250]), (2, 128, [500], [64]), (1, 64, [2000], [80]),
+           (1, 64, [4000] + [0] * 26, [64] * 27)]
+
+
+@pytest.mark.parametrize("q8", [False, True], ids=["f16", "q8"])
+@pytest.mark.parametrize("L,D,ctx,rows", PROMPTS, ids=lambda x: f"{len(x)}x{x[0]}" if isinstance(x, list) else str(x))
+def test_noalloc_equals_step_on_prompts(gpu, L, D, ctx, rows, q8):
+    """Both entry points choose the same query groups, whatever fits the one
+    that allocates nothing: the same bits."""
+    C_ = 768
+    n_ctx = max(c + r for c, r in zip(ctx, rows))
+    opts = na.BatchOpts(n_layer=L, n_head=C_ // D, head_dim=D, kv_blocks=sum((c + r) // 16 + 1 for c, r in zip(ctx, rows)),
+                        max_seqs=len(ctx), n_ctx=n_ctx, max_rows=2048, q8=q8)
+    a, b = na.PagedKv(opts), na.PagedKv(opts)
+    g = torch.Generator(device="cuda").manual_seed(sum(rows))
+    for s, c in enumerate(ctx):
+        for kv in (a, b):
+            assert kv.add_seq() == s
+        for p0 in range(0, c, 2048):
+            n = min(c, p0 + 2048) - p0
+            k, v = (torch.randn((L, n, C_), device="cuda", generator=g) for _ in range(2))
+            for kv in (a, b):
+                kv.reserve(s, p0 + n)
+                kv.append([(s, p0 + i) for i in range(n)], k, v)
+                kv.commit(s, n)
+    lib = _abi.lib()
+    work = [(s, r, r) for s, r in enumerate(rows)]
+    n = sum(rows)
+    q, k, v = (torch.randn((L, n, C_), device="cuda", generator=g) for _ in range(3))
+    out_a, out_b = (torch.full((L, n, C_), float("nan"), device="cuda") for _ in range(2))
+    say(f"no-alloc prompts: {L} layers x {D}, {len(rows)} sequences, {n} rows")
+    assert call(a, lib.ni_kv_step, work, q, k, v, out_a, 0) == 0, lib.ni_kv_last_error(a.handle).decode()
+    assert call(b, lib.ni_kv_step_noalloc, work, q, k, v, out_b, 0) == 0, lib.ni_kv_last_error(b.handle).decode()
+    torch.cuda.synchronize()
+    assert torch.isfinite(out_a).all()
+    assert torch.equal(out_a, out_b)
+    a.close()
+    b.close()
+
+
 def test_noalloc_limits(gpu):
     lib = _abi.lib()
     # A plan over 32 KB: 64 sequences of 2048 positions list 64 x 129 page ids.
