@@ -102,6 +102,33 @@ __device__ __forceinline__ void merge_state(float& m, float& l, float (&o)[N], f
 // empty states is 1 (not NaN); masked scores are -inf and weigh 0.
 constexpr float kMinScore = -1e30f;
 
+// The states (m, l, o) of W waves for one output of a row, wave w's at red +
+// w * stride: weighed by exp2(m - M) and added pairwise, as a tree (a chain
+// over 16 waves rounds each sum 15 times, the tree 4).
+template <int W>
+__device__ __forceinline__ void merge_waves(const float* red, uint32_t stride, uint32_t d, float& M, float& L,
+                                            float& O) {
+    float l[W], o[W];
+    M = red[0];
+#pragma unroll
+    for (int w = 1; w < W; w++) M = fmaxf(M, red[w * stride]);
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+        const float wt = fast_exp2(red[w * stride] - M);
+        l[w] = red[w * stride + 1] * wt;
+        o[w] = red[w * stride + 2 + d] * wt;
+    }
+#pragma unroll
+    for (int n = 1; n < W; n *= 2)
+#pragma unroll
+        for (int w = 0; w + n < W; w += 2 * n) {
+            l[w] += l[w + n];
+            o[w] += o[w + n];
+        }
+    L = l[0];
+    O = o[0];
+}
+
 // A plan passed with the kernel arguments (N > 0) or left in device memory
 // (N == 0: the launch struct's `plan` pointer).  Arguments live in the
 // read-only kernarg segment; the kernels index it in place.
@@ -574,12 +601,12 @@ __global__ __launch_bounds__(64 * W, W == 8 ? kWideMinWaves : 1) void attn_split
                 const half8_t kh = __builtin_bit_cast(half8_t, cur.k[b][i]);
 #pragma unroll
                 for (int r = 0; r < NQ; r++) {
-                    float acc = 0.f;
+                    float acc[2] = {0.f, 0.f};
                     if (r < (int)it.nq) {
 #pragma unroll
-                        for (int e = 0; e < 8; e++) acc = fmaf(q[r][e], static_cast<float>(kh[e]), acc);
+                        for (int e = 0; e < 8; e++) acc[e / 4] = fmaf(q[r][e], static_cast<float>(kh[e]), acc[e / 4]);
                     }
-                    s[r][b][i] = key_sum<LPK>(acc);
+                    s[r][b][i] = key_sum<LPK>(acc[0] + acc[1]);
                 }
             }
         }
@@ -607,20 +634,26 @@ __global__ __launch_bounds__(64 * W, W == 8 ? kWideMinWaves : 1) void attn_split
             const float mn = fmaxf(m[r], mb);
             const float alpha = fast_exp2(m[r] - mn);
             m[r] = mn;
-            l[r] *= alpha;
-#pragma unroll
-            for (int e = 0; e < 8; e++) o[r][e] *= alpha;
+            // The iteration's keys are added up first, then to the sums so far
+            // (and the score above in two parts): whole launches add more keys
+            // per lane than partitions do (1 row of 901 keys, 16 waves: 1.7e-7
+            // of the norm against 64 bits added one by one, 1.5e-7 so, 1.6e-7 in
+            // partitions one by one; the same time).
+            float ps = 0.f, t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int b = 0; b < PB; b++) {
 #pragma unroll
                 for (int i = 0; i < LPP; i++) {
                     const float p = fast_exp2(s[r][b][i] - mn);
-                    l[r] += p;
+                    ps += p;
                     const half8_t vh = __builtin_bit_cast(half8_t, cur.v[b][i]);
 #pragma unroll
-                    for (int e = 0; e < 8; e++) o[r][e] = fmaf(p, static_cast<float>(vh[e]), o[r][e]);
+                    for (int e = 0; e < 8; e++) t[e] = fmaf(p, static_cast<float>(vh[e]), t[e]);
                 }
             }
+            l[r] = fmaf(l[r], alpha, ps);
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[r][e] = fmaf(o[r][e], alpha, t[e]);
         }
         cur = nxt;
     }
@@ -656,16 +689,8 @@ __global__ __launch_bounds__(64 * W, W == 8 ? kWideMinWaves : 1) void attn_split
     // group's only partition, else the partial (m, l, o) for the merge kernel.
     for (uint32_t t = threadIdx.x; t < it.nq * D; t += 64 * W) {
         const uint32_t r = t / D, d = t - r * D;
-        float M = red[0][r][0];
-#pragma unroll
-        for (int w = 1; w < W; w++) M = fmaxf(M, red[w][r][0]);
-        float L = 0.f, O = 0.f;
-#pragma unroll
-        for (int w = 0; w < W; w++) {
-            const float wt = fast_exp2(red[w][r][0] - M);
-            L += red[w][r][1] * wt;
-            O += red[w][r][2 + d] * wt;
-        }
+        float M, L, O;
+        merge_waves<W>(red[0][r], NQ * (D + 2), d, M, L, O);
         if (it.part_slot == kNoSlot) {
             a.out[(int64_t)lay * a.out_layer_stride + (int64_t)(it.row0 + r) * a.out_row_stride + head * D + d] = O / L;
         } else {
@@ -787,16 +812,8 @@ __global__ __launch_bounds__(64 * W) void attn_rows_kernel(const RowsLaunch a) {
     }
     __syncthreads();
     for (uint32_t d = threadIdx.x; d < (uint32_t)D; d += 64 * W) {
-        float M = red[0][0];
-#pragma unroll
-        for (int w = 1; w < W; w++) M = fmaxf(M, red[w][0]);
-        float L = 0.f, O = 0.f;
-#pragma unroll
-        for (int w = 0; w < W; w++) {
-            const float wt = fast_exp2(red[w][0] - M);
-            L += red[w][1] * wt;
-            O += red[w][2 + d] * wt;
-        }
+        float M, L, O;
+        merge_waves<W>(red[0], D + 2, d, M, L, O);
         a.out[(int64_t)i * a.out_stride + h * D + d] = O / L;
     }
 }
@@ -1003,12 +1020,19 @@ __global__ __launch_bounds__(64 * W) void attn_q8_kernel(const AttnLaunch a, con
         for (int b = 0; b < PB; b++) {
 #pragma unroll
             for (int i = 0; i < LPP; i++) {
-                float acc = 0.f;
+                // (four sums, as in attn_split_kernel; launches of kWaves waves,
+                // bound by these conversions, one: 85.3 against 89 us for 64
+                // sequences of 32..767 keys, 12 layers)
+                float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int w = 0; w < 4; w++)
 #pragma unroll
-                    for (int j = 0; j < 4; j++) acc = fmaf(q[4 * w + j], i8f(cur.k[b][i][w], j), acc);
-                s[b][i] = key_sum<LPK>(acc) * cur.ks[b][i];
+                    for (int j = 0; j < 4; j++) {
+                        float& x = acc[W == kWaves ? 0 : w];
+                        x = fmaf(q[4 * w + j], i8f(cur.k[b][i][w], j), x);
+                    }
+                if constexpr (W != kWaves) acc[0] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+                s[b][i] = key_sum<LPK>(acc[0]) * cur.ks[b][i];
                 const uint32_t key = (pg + b) * kPage + i * KPL + kl;
                 if (key > it.pos0 || key >= it.kv_end) {
                     s[b][i] = -INFINITY;
@@ -1063,16 +1087,8 @@ __global__ __launch_bounds__(64 * W) void attn_q8_kernel(const AttnLaunch a, con
     }
     __syncthreads();
     for (uint32_t d = threadIdx.x; d < D; d += 64 * W) {
-        float M = red[0][0];
-#pragma unroll
-        for (int w = 1; w < W; w++) M = fmaxf(M, red[w][0]);
-        float L = 0.f, O = 0.f;
-#pragma unroll
-        for (int w = 0; w < W; w++) {
-            const float wt = fast_exp2(red[w][0] - M);
-            L += red[w][1] * wt;
-            O += red[w][2 + d] * wt;
-        }
+        float M, L, O;
+        merge_waves<W>(red[0], D + 2, d, M, L, O);
         if (it.part_slot == kNoSlot) {
             a.out[(int64_t)lay * a.out_layer_stride + (int64_t)it.row0 * a.out_row_stride + head * D + d] = O / L;
         } else {
@@ -1545,9 +1561,9 @@ __device__ __forceinline__ uint32_t tile_chunk(uint32_t key, uint32_t q) {
 }
 typedef __fp16 v4fp16_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
 #define NI_LDS(p) ((__attribute__((address_space(3))) void*)(p))
-// p in [0, 1] enters PV scaled by 2^14 (through the exponent reference:
-// exp2(s - (m - 14))), so that p down to ~4e-9 is a normal f16.
-constexpr float kPUnscale = 1.f / 16384.f, kLog2PScale = 14.f;
+// p in [0, 1] enters PV scaled by 2^14, so that p down to ~4e-9 is a normal
+// f16.
+constexpr float kPScale = 16384.f, kPUnscale = 1.f / kPScale;
 
 // Groups of 2..16 queries of one sequence (speculative verify, prefill
 // chunks) on matrix cores: one wave per page walks S^T = K Q^T (16 keys x 16
@@ -1829,16 +1845,19 @@ __global__ __launch_bounds__(64 * W, D == 64 ? kMfmaMinWaves : 1) void attn_mfma
                 vinv = 1.f / vm;
             }
         }
-        // Weights scaled by 2^14 through the exponent reference, so lsum
-        // is in those units too; Q8 weighs p by vs / vref before the split.
-        const float mref = mn - kLog2PScale;
+        // Weights scaled by 2^14, so lsum is in those units too; Q8 weighs p
+        // by vs / vref before the split.  Scaled after the exponential: in the
+        // exponent (s - (m - 14)) the largest weights' arguments, near 14, are
+        // rounded 2^-21 off, and the reference itself as much in each wave
+        // (5 rows of 900 keys: 2.9e-7 of the norm against 64 bits, 4 multiplies
+        // a page cost nothing measurable).
         half4_t ph[PB], pl[PB];
         float ps = 0.f;
 #pragma unroll
         for (int b = 0; b < PB; b++) {
             float p[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) p[j] = fast_exp2(s[b][j] - mref);
+            for (int j = 0; j < 4; j++) p[j] = fast_exp2(s[b][j] - mn) * kPScale;
             ps += (p[0] + p[1]) + (p[2] + p[3]);
             if constexpr (Q8) {
 #pragma unroll
@@ -1916,16 +1935,8 @@ __global__ __launch_bounds__(64 * W, D == 64 ? kMfmaMinWaves : 1) void attn_mfma
     __syncthreads();
     for (uint32_t t = threadIdx.x; t < it.nq * D; t += 64 * W) {
         const uint32_t r = t / D, d = t - r * D;
-        float M = red[0][r][0];
-#pragma unroll
-        for (int w = 1; w < W; w++) M = fmaxf(M, red[w][r][0]);
-        float L = 0.f, O = 0.f;
-#pragma unroll
-        for (int w = 0; w < W; w++) {
-            const float wt = fast_exp2(red[w][r][0] - M);
-            L += red[w][r][1] * wt;
-            O += red[w][r][2 + d] * wt;
-        }
+        float M, L, O;
+        merge_waves<W>(red[0][r], NQ * (D + 2), d, M, L, O);
         if (it.part_slot == kNoSlot) {
             a.out[(int64_t)lay * a.out_layer_stride + (int64_t)(it.row0 + r) * a.out_row_stride + head * D + d] = O / L;
         } else {
@@ -2252,16 +2263,8 @@ __global__ __launch_bounds__(64 * W) void attn_rows_tile_kernel(const RowsLaunch
     __syncthreads();
     for (uint32_t u = threadIdx.x; u < nq * D; u += 64 * W) {
         const uint32_t row = u / D, d = u - row * D;
-        float M = red[0][row][0];
-#pragma unroll
-        for (int w = 1; w < W; w++) M = fmaxf(M, red[w][row][0]);
-        float L = 0.f, O = 0.f;
-#pragma unroll
-        for (int w = 0; w < W; w++) {
-            const float wt = fast_exp2(red[w][row][0] - M);
-            L += red[w][row][1] * wt;
-            O += red[w][row][2 + d] * wt;
-        }
+        float M, L, O;
+        merge_waves<W>(red[0][row], kRowsTile * (D + 2), d, M, L, O);
         a.out[(int64_t)(q0 + row) * a.out_stride + h * D + d] = O / L;
     }
 }
