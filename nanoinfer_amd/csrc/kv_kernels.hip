@@ -2051,13 +2051,15 @@ __device__ __forceinline__ void wait_tiles(uint32_t ahead) {
 // the result against 64 bits at 1024 keys; one accumulator throughout 2.6e-7):
 // a score adds D/4 products of 4 dims as a tree, and the keys go to 4
 // accumulators by key % 4.  The exponent reference follows the running max
-// only past kRefSlack (weights up to 2^8, f32 throughout).
+// only past kRefSlack; the weights, up to 2^8 by it, are scaled back to 1 at
+// most, so that sums of large V stay finite as they do on attn_rows_kernel.
 //
 // Rows past the last key repeat it (nothing past it is read).  A key hidden
 // from some query of a tile may hold infinities or NaN, which 0 * V would turn
 // into NaN in that query's sum: tiles with hidden keys check their V values
 // and, where one is not finite, add their rows one by one instead.
 constexpr int kRowsTile = 16;  // keys per tile, queries per workgroup
+constexpr float kRefUnscale = 1.f / 256.f;  // 2^-kRefSlack
 
 template <int D, int W>
 __global__ __launch_bounds__(64 * W) void attn_rows_tile_kernel(const RowsLaunch a) {
@@ -2205,7 +2207,7 @@ __global__ __launch_bounds__(64 * W) void attn_rows_tile_kernel(const RowsLaunch
                     for (int c = 0; c < 4; c++) o[n][g][c] *= alpha;
         }
 #pragma unroll
-        for (int e = 0; e < 4; e++) s[e] = fast_exp2(s[e] - m);
+        for (int e = 0; e < 4; e++) s[e] = fast_exp2(s[e] - m) * kRefUnscale;
         l += (s[0] + s[1]) + (s[2] + s[3]);
         if (masked) {
             bool bad = false;

@@ -90,3 +90,20 @@ def test_row_kernel_wave_counts(gpu, h, d, nq, p0):
     want, bound = exact(*(x.cpu().numpy() for x in (q, k, v)), p0, h, d)
     got = na.attention(q, k, v, nq, p0, h, d).cpu().numpy()
     assert (np.abs(got - want) <= bound).all()
+
+
+@pytest.mark.parametrize("h,d,nq,p0", [(12, 64, 256, 0), (12, 64, 640, 0), (32, 128, 100, 5)])
+def test_large_values_stay_finite(gpu, h, d, nq, p0):
+    """A later key's score 7.5 (base 2) above the first 16 keys': weights
+    relative to those would be 181, times 60 keys or more of V up to 2e35 past
+    f32's 3.4e38, though the result is their mean."""
+    g = torch.Generator(device="cuda").manual_seed(7)
+    c, n = h * d, p0 + nq
+    a = math.sqrt(7.5 * math.log(2) / math.sqrt(d))
+    q, k = (torch.full((r, c), a, device="cuda") for r in (nq, n))
+    k[:16] = 0
+    v = (1 + torch.rand((n, c), device="cuda", generator=g)) * 1e35
+    want, bound = exact(*(x.cpu().numpy() for x in (q, k, v)), p0, h, d)
+    got = na.attention(q, k, v, nq, p0, h, d).cpu().numpy()
+    assert np.isfinite(got).all()
+    assert (np.abs(got - want) <= bound).all()
