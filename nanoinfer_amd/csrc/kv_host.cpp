@@ -517,89 +517,7 @@ struct Cut {
     }
 };
 
-// The automatic cut (split_tokens 0).  Splitting costs a merge launch (~5-7
-// us) and the partials' round trip, so it pays only when the unsplit items
-// cannot keep the GPU busy: 256 CUs hold 1024 workgroups at once, and with >=
-// 2048 of them, sorted longest first, the tail is short -- only items longer
-// than kLongItem keys are split then.  Below that, the largest of
-// 1024/512/256/128 tokens that yields >= 2048 workgroups.
-// At head_dim 64, launches of single rows or of groups within one matrix
-// tile below that are not split either: several waves of one workgroup
-// share each item's pages and merge in LDS, no partials, no merge launch
-// (us per launch, split and merged against one workgroup per item):
-// * single rows: kWideWaves waves (Q8: kWideWavesQ8), kSoloWaves while
-//   every unit has a CU of its own and the items are long enough to keep
-//   16 waves busy, kWaves up to kNarrowKeys keys, where waves of 2 pages
-//   cover an item at once.  12 layers x 12 heads: 1 sequence of 150 keys
-//   7.1 / 3.9, 300 7.9 / 5.2, 517 9.2 / 6.6, 1000 11.5 / 9.1, 3000 24.3 /
-//   20.5, 3 of 1000 24.3 / 19.0; Q8 517 9.9 / 7.0, 3 of 1000 21.0 / 13.2.
-// * groups: kWideWaves waves below kWideMinUnits units (12 layers, 5 rows of
-//   300 keys 8.2 / 5.8, 1000 13.7 / 10.1), from there on, where two such
-//   workgroups no longer fit each CU, kWaves (4 x U[64,1000] 23.2 -> 19.5,
-//   13 41.9 -> 37.0).
-// Below kWholeMinUnits units that holds up to kShortItem keys only: longer
-// items fill the GPU faster in partitions (one layer of 12 heads: 1
-// sequence of 2000 keys 8.1 / 12.5, 4 of 2000 11.4 / 13.4, 16 of 2000 24.1 /
-// 18.8).
-// Prefill groups (more rows than one matrix tile, in a launch of their
-// own) are split automatically only past kLongItem keys: each of their
-// workgroups already carries 64 queries, and splitting them to fill the
-// GPU cost more than it gained (prompt steps, every row queried, no split
-// against the fill choice: one launch per layer 16 x 512 rows 611 against
-// 753 us, 4 x 512 286 against 436, 1 x 512 254 against 305; all layers 1 x
-// 512 45 against 67 us, 4 x 512 146 against 167, 2 x 512 and 8 x 256 the
-// same).
-constexpr uint32_t kLongItem = 4096;
-Cut auto_cut(const ni_kv* kv, const std::vector<Group>& groups, uint32_t n_lay) {
-    constexpr uint64_t kFillWorkgroups = 2048;
-    constexpr uint64_t kWideMinUnits = 512;
-    constexpr uint64_t kWholeMinUnits = 96;
-    constexpr uint32_t kNarrowKeys = 128, kSoloKeys = 384, kSoloKeysQ8 = 640;
-    static const uint32_t kChoices[] = {1024, 512, 256, 128};
-    Cut cut{kLongItem, kLongItem, 0};
-    const uint64_t per_unit = (uint64_t)n_lay * kv->o.n_head;
-    const uint64_t units = (uint64_t)groups.size() * per_unit;
-    constexpr uint32_t kShortItem = 1280;  // keys (a 1024-token context and its new rows)
-    const uint32_t whole_keys = units >= kWholeMinUnits ? kLongItem : kShortItem;
-    bool single = true, tiles = true;  // every group one row; every group within one matrix tile
-    uint32_t max_keys = 0;
-    for (const Group& g : groups) {
-        single &= g.nq == 1;
-        tiles &= g.nq <= kMfmaTile && !g.pre;
-        max_keys = std::max(max_keys, g.pos0 + g.nq);
-    }
-    if (units >= kFillWorkgroups) {
-        cut.part = kLongItem;
-    } else if (tiles && kv->o.head_dim == 64 &&
-               (units >= (single ? kWideMinUnits : kWideMinUnits / 2) || max_keys <= whole_keys)) {
-        cut.part = kLongItem;
-        const uint32_t solo_keys = is_q8(kv->o) ? kSoloKeysQ8 : kSoloKeys;
-        if (!single)
-            cut.wide = units < kWideMinUnits ? 1u : 0u;
-        else if (units >= kWideMinUnits || max_keys > kNarrowKeys)
-            cut.wide = units <= device_cus() && max_keys > solo_keys ? 2u : 1u;
-    } else if (n_lay == 1 && max_keys <= kShortItem) {
-        // One layer per launch and no item past kShortItem keys: the
-        // merge launch a split needs costs more than the fill it buys
-        // (decode rows of 4..32 sequences with contexts U[64,1024]: 213-240
-        // against 251-284 us per step of 12 such launches; 8 x 1024 keys
-        // 208 against 246; from 2048 keys the split wins, 4 x 2048 242
-        // against 285, 4 x 4096 246 against 524, and 16 x U[1024,2048]
-        // 262 against 273).
-        cut.part = kLongItem;
-    } else {
-        cut.part = kChoices[3];
-        for (uint32_t c : kChoices) {
-            uint64_t items = 0;
-            for (const Group& g : groups) items += ((uint64_t)g.pos0 + g.nq + c - 1) / c;
-            if (items * per_unit >= kFillWorkgroups) {
-                cut.part = c;
-                break;
-            }
-        }
-    }
-    return cut;
-}
+constexpr uint32_t kLongItem = 4096;  // keys: the automatic cut splits longer items whatever the launch
 
 // Whether ni_kv_step_noalloc takes a launch cut this way (its plan inline, its
 // partials in the scratch array).  ni_kv_step asks too, so that both run the
@@ -620,16 +538,129 @@ bool noalloc_takes(const ni_kv* kv, const std::vector<Group>& groups, const Cut&
     }
     size_t bytes = 0;
     auto add = [&](size_t n, size_t size) { bytes = align_up(bytes + n * size, kAlign); };
-    add(kv->plan.app.size(), sizeof(AppendEntry));
+    const bool streams = kv->plan.fused && kv->o.head_dim == 64 && nq_tile == 1 && (!is_q8(kv->o) || cut.wide);
+    if (!streams) add(kv->plan.app.size(), sizeof(AppendEntry));
     add(kv->plan.orphans.size(), sizeof(AppendEntry));
     for (int p = 0; p < 2; p++) {
         add(items[p], sizeof(AttnItem));
         add(merges[p], sizeof(MergeItem));
     }
     add(n_table, sizeof(uint32_t));
-    if (cut.wide) add(items[0] * lh, sizeof(uint16_t));  // the order of its units
+    const uint64_t units = items[0] * lh;
+    if (cut.wide && units > device_cus() && (nq_tile > 1 || units >= 512)) add(units, sizeof(uint16_t));  // their order
     const size_t partials = (slots[0] * nq_tile + slots[1] * kPrefillRows) * lh * (kv->o.head_dim + 2) * sizeof(float);
     return bytes <= kInlinePlanBytes && partials <= kScratchBytes;
+}
+
+// The automatic cut (split_tokens 0).  Splitting costs a merge launch (~5-7
+// us) and the partials' round trip, so it pays only when the unsplit items
+// cannot keep the GPU busy: 256 CUs hold 1024 workgroups at once, and with >=
+// 2048 of them, sorted longest first, the tail is short -- only items longer
+// than kLongItem keys are split then.  Below that, the largest of
+// 1024/512/256/128 tokens that yields >= 2048 workgroups.
+// At head_dim 64, launches of single rows or of groups within one matrix
+// tile below that may run whole: several waves of one workgroup share each
+// item's pages and merge in LDS, no partials, no merge launch.  They wait for
+// their longest item, partitions for the launch's keys spread over the GPU, so
+// the line between the two is the longest item's keys against `mean`, the
+// launch's keys per CU (us per launch, partitions / whole):
+// * single rows, a CU for every unit (kSoloWaves waves, kWideWaves up to
+//   kSoloKeys): up to kShortItem keys (12 layers x 12 heads: 150 keys 7.1 / 3.9,
+//   517 9.2 / 6.6, 1000 11.5 / 9.1; 2 layers, 1280 keys 8.9 / 8.4) or 1280 + 1.75
+//   mean (Q8: 2), 3072 at most on f16, where the longer sums begin to show
+//   (one layer, 16 of 2000 keys 24.2 / 17.4, 8 of 3000 20.4 / 19.1, 8 of 4090
+//   25.0 / 27.0; one of 2000 and 7 of 100 9.7 / 9.7, one of 4090 and 7 of 100
+//   10.8 / 15.4, Q8 11.4 / 18.1).
+// * single rows, two units on some CUs (kWideWaves; Q8 kWideWavesQ8): up to
+//   kShortItem or 1500 + 0.43 mean, 2048 at most (Q8 1536: as above) (12 layers,
+//   3 of 1500 keys 31.4 / 27.2; 2 of 2000 29.2 / 29.4; one layer, one of 2000 and
+//   31 of 100 10.6 / 12.6, one of 4090 and 41 of 100 12.6 / 27.6, Q8 13.9 / 29.4).
+// * groups (kWideWaves) below kWideMinUnits / 2 units: up to 700 + (1.6 + 0.04
+//   per row of the largest group) mean (Q8: 1.25), one layer per launch up to
+//   kShortItem (12 layers, 5 rows of 300 keys 8.2 / 5.8, 1000 13.7 / 10.1; 2
+//   layers, 600 keys 9.3 / 8.1, 1280 10.0 / 12.2; one layer, 16 of 2000 28.2 /
+//   19.4, one of 2000 and 7 of 100 11.2 / 15.9).
+// From kWideMinUnits units on (groups: half as many) always.  kNarrowKeys keys
+// and less take kWaves waves of 2 pages, which cover an item at once.
+//
+// Groups from kWideMinUnits units on take kWaves waves where that is faster:
+// twice the chain of the longest item, but four workgroups per CU instead of
+// two.  Measured for kWideWaves / kWaves: the longest item's chain 4.3 + 6.4 / 5
+// + 10.6 per 1000 keys, 5.5 per round of workgroups / not reached, 11.6 / 10.8 per
+// 1000 keys of mean (5 rows, 12 layers: 8 x U[64,1000] 27.9 / 25.5, 13 45.1 / 42.0;
+// one of 700 and 3 of 100 9.8 / 12.2, 7 of 100 15.8 / 13.2; one of 2000 and 7 of
+// 100 20.0 / 27.2; one layer, one of 4090 and 159 of 100 32.2 / 50.9).
+// Prefill groups (more rows than one matrix tile, in a launch of their
+// own) are split automatically only past kLongItem keys: each of their
+// workgroups already carries 64 queries, and splitting them to fill the
+// GPU cost more than it gained (prompt steps, every row queried, no split
+// against the fill choice: one launch per layer 16 x 512 rows 611 against
+// 753 us, 4 x 512 286 against 436, 1 x 512 254 against 305; all layers 1 x
+// 512 45 against 67 us, 4 x 512 146 against 167, 2 x 512 and 8 x 256 the
+// same).
+Cut auto_cut(const ni_kv* kv, const std::vector<Group>& groups, uint32_t n_lay, size_t n_table) {
+    constexpr uint64_t kFillWorkgroups = 2048;
+    constexpr uint64_t kWideMinUnits = 512;
+    constexpr uint32_t kShortItem = 1280;  // keys (a 1024-token context and its new rows)
+    constexpr uint32_t kNarrowKeys = 128, kSoloKeys = 384, kSoloKeysQ8 = 640;
+    static const uint32_t kChoices[] = {1024, 512, 256, 128};
+    const Cut whole{kLongItem, kLongItem, 0};
+    const uint64_t per_unit = (uint64_t)n_lay * kv->o.n_head;
+    const uint64_t units = (uint64_t)groups.size() * per_unit;
+    if (units >= kFillWorkgroups) return whole;
+    bool single = true, tiles = true;  // every group one row; every group within one matrix tile
+    uint32_t max_keys = 0, max_nq = 0;
+    uint64_t keys = 0;
+    for (const Group& g : groups) {
+        single &= g.nq == 1;
+        tiles &= !g.prefill();
+        max_nq = std::max(max_nq, g.nq);
+        max_keys = std::max(max_keys, g.keys());
+        keys += g.keys();
+    }
+    Cut wide = whole;
+    const bool may_whole = tiles && kv->o.head_dim == 64 &&
+                           (units >= (single ? kWideMinUnits : kWideMinUnits / 2) || max_keys <= kLongItem);
+    if (may_whole) {
+        const bool q8 = is_q8(kv->o), solo = units <= device_cus();
+        const double mean = (double)keys * per_unit / device_cus();
+        double line = kLongItem;
+        if (!single) {
+            const double us8 = std::max({4.3 + 6.4e-3 * max_keys, 5.5 * ((units + 511) / 512), 11.6e-3 * mean});
+            const double us4 = std::max(5 + 10.6e-3 * max_keys, 10.8e-3 * mean);
+            wide.wide = units < kWideMinUnits || us8 <= us4 ? 1u : 0u;
+            line = 700 + ((q8 ? 1.25 : 1.6) + 0.04 * max_nq) * mean;
+            if (n_lay == 1) line = std::max(line, (double)kShortItem);
+        } else {
+            if (units >= kWideMinUnits || max_keys > kNarrowKeys)
+                wide.wide = solo && max_keys > (q8 ? kSoloKeysQ8 : kSoloKeys) ? 2u : 1u;
+            line = solo ? std::min(1280 + (q8 ? 2. : 1.75) * mean, q8 ? 4096. : 3072.)
+                        : std::min(1500 + 0.43 * mean, q8 ? 1536. : 2048.);
+            line = std::max(line, (double)kShortItem);
+        }
+        if (units >= (single ? kWideMinUnits : kWideMinUnits / 2) || max_keys <= line) return wide;
+    }
+    // One layer per launch and no item past kShortItem keys: the merge
+    // launch a split needs costs more than the fill it buys (decode rows of
+    // 4..32 sequences with contexts U[64,1024]: 213-240 against 251-284 us per
+    // step of 12 such launches; 8 x 1024 keys 208 against 246; from 2048 keys
+    // the split wins, 4 x 2048 242 against 285, 4 x 4096 246 against 524, and 16
+    // x U[1024,2048] 262 against 273).
+    if (n_lay == 1 && max_keys <= kShortItem) return whole;
+    Cut cut = whole;
+    cut.part = kChoices[3];
+    for (uint32_t c : kChoices) {
+        uint64_t items = 0;
+        for (const Group& g : groups) items += ((uint64_t)g.keys() + c - 1) / c;
+        if (items * per_unit >= kFillWorkgroups) {
+            cut.part = c;
+            break;
+        }
+    }
+    // (whole where ni_kv_step_noalloc takes only that)
+    const bool fits = !may_whole || noalloc_takes(kv, groups, cut, n_lay, n_table) ||
+                      !noalloc_takes(kv, groups, wide, n_lay, n_table);
+    return fits ? cut : wide;
 }
 
 // Attention part of a plan: group the query rows, cut each group's keys into
@@ -654,10 +685,10 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
     }
     Cut cut{split_tokens, split_tokens, 0};
     if (split_tokens == 0) {
-        cut = auto_cut(kv, groups, n_lay);
+        cut = auto_cut(kv, groups, n_lay, n_table);
         if (prefill && small_groups(kv, n_lay)) {
             std::vector<Group> tiles = form_groups(qr, max_group_rows(kv));
-            const Cut c = auto_cut(kv, tiles, n_lay);
+            const Cut c = auto_cut(kv, tiles, n_lay, n_table);
             if (noalloc_takes(kv, tiles, c, n_lay, n_table) || !noalloc_takes(kv, groups, cut, n_lay, n_table)) {
                 groups.swap(tiles);
                 cut = c;

@@ -117,3 +117,40 @@ def test_groups(gpu, oracle_lib, n_seqs, nq, ctx):
             for s, n in zip(seqs, base):
                 m.kv.truncate(s, n)
     m.kv.close()
+
+
+@pytest.mark.parametrize("q8", [False, True], ids=["f16", "q8"])
+@pytest.mark.parametrize("n_layer,nq,ctx,whole", [
+    (1, 1, [4090] + [100] * 7, False), (1, 1, [4090] + [100] * 31, False), (12, 1, [4090, 100], False),
+    (1, 1, [2000] * 16, True), (12, 1, [1500], True), (1, 1, [1280] + [100] * 7, True), (12, 1, [1280] * 2, True),
+    (1, 5, [2000] + [100] * 7, False), (2, 16, [1280], False), (1, 5, [4090] + [100] * 7, False),
+    (1, 5, [2000] * 16, True), (12, 5, [1500], True), (1, 16, [1280] + [100] * 7, True)],
+    ids=lambda x: f"{len(x)}x{x[0]}" if isinstance(x, list) else str(x))
+def test_long_items_run_whole_beside_enough_others(gpu, n_layer, nq, ctx, whole, q8):
+    """A launch waits for its longest whole item: one long context among short
+    ones goes in partitions (and a merge launch), as many as it fills the GPU
+    with stay whole.  The results agree with partitions of 256 keys (f32 sums
+    or f16 pairs in another order: 4e-6 of the norm)."""
+    kv = na.PagedKv(na.BatchOpts(n_layer=n_layer, n_head=12, head_dim=64, q8=q8, kv_blocks=sum(c // 16 + 1 for c in ctx),
+                                 max_seqs=len(ctx), n_ctx=max(ctx), max_rows=2048))
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rows = []
+    for c in ctx:
+        s = kv.add_seq()
+        kv.reserve(s, c)
+        for p in range(0, c, 2048):
+            n = min(c, p + 2048) - p
+            k, v = (torch.randn((n_layer, n, 768), device="cuda", generator=g) for _ in range(2))
+            kv.append([(s, p + i) for i in range(n)], k, v)
+        kv.commit(s, c)
+        rows += [(s, c - nq + i) for i in range(nq)]
+    q = torch.randn((n_layer, len(rows), 768), device="cuda", generator=g)
+    kv.profile([2])
+    got = kv.attention(q, rows)
+    torch.cuda.synchronize()
+    _, n_merge = kv.profile_read(2)
+    kv.profile([])
+    assert n_merge == (0 if whole else 1)
+    want = kv.attention(q, rows, split_tokens=256).double()
+    assert (got - want).norm() / want.norm() < 4e-6
+    kv.close()

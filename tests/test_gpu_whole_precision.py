@@ -40,7 +40,8 @@ def _exact(q, k, v):
 @pytest.mark.parametrize("seqs,nq,keys,q8,bound", [
     (1, 1, 150, False, 1.40e-7), (1, 1, 517, False, 1.51e-7), (1, 1, 901, False, 1.64e-7), (1, 1, 1270, False, 1.77e-7),
     (1, 1, 3000, False, 1.84e-7), (3, 1, 900, False, 1.62e-7), (3, 1, 1270, False, 1.78e-7),
-    (1, 1, 517, True, 0.94e-7), (1, 1, 901, True, 0.91e-7), (3, 1, 1270, True, 0.76e-7), (1, 1, 3500, True, 0.75e-7),
+    (1, 1, 517, True, 0.94e-7), (1, 1, 901, True, 0.91e-7), (3, 1, 1270, True, 0.76e-7), (3, 1, 1500, True, 0.78e-7),
+    (3, 1, 2000, False, 1.79e-7),  (1, 1, 3500, True, 0.75e-7),
     (1, 5, 300, False, 2.57e-7), (1, 5, 900, False, 2.65e-7), (1, 16, 900, False, 2.66e-7),
     (6, 5, 900, False, 2.92e-7), (13, 5, 700, False, 2.84e-7), (1, 5, 900, True, 0.93e-7), (6, 5, 900, True, 1.07e-7)])
 def test_error_of_whole_launches(gpu, seqs, nq, keys, q8, bound):

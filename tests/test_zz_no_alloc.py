@@ -194,6 +194,29 @@ def test_noalloc_equals_step_on_prompts(gpu, L, D, ctx, rows, q8):
     b.close()
 
 
+def test_noalloc_takes_long_rows_whole(gpu):
+    """19 rows of 4090 keys, one layer: in partitions of 256 keys a plan past
+    32 KB, whole 20 KB.  Both entry points run it whole."""
+    opts = na.BatchOpts(n_layer=1, n_head=12, head_dim=64, kv_blocks=19 * 257, max_seqs=19, n_ctx=4096, max_rows=64)
+    a, b = na.PagedKv(opts), na.PagedKv(opts)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    work = [(s, 1, 1) for s in range(19)]
+    q, k, v = (torch.randn((1, 19, 768), device="cuda", generator=g) for _ in range(3))
+    outs = []
+    lib = _abi.lib()
+    for kv, fn in ((a, lib.ni_kv_step), (b, lib.ni_kv_step_noalloc)):
+        for s in range(19):
+            assert kv.add_seq() == s
+            kv.reserve(s, 4089)
+            kv.commit(s, 4089)  # pages hold zeros: never written
+        outs.append(torch.full_like(q, float("nan")))
+        assert call(kv, fn, work, q, k, v, outs[-1], 0) == 0, lib.ni_kv_last_error(kv.handle).decode()
+    torch.cuda.synchronize()
+    assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
+    a.close()
+    b.close()
+
+
 def test_noalloc_limits(gpu):
     lib = _abi.lib()
     # A plan over 32 KB: 64 sequences of 2048 positions list 64 x 129 page ids.
