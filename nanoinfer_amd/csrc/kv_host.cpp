@@ -423,62 +423,6 @@ void balance_prefill_units(Plan& P, uint32_t n_lay, uint32_t n_head, uint64_t C,
     deal_units(cost, lh, C, R, rem, P.porder);
 }
 
-// Whether a launch of prompt chunks runs faster as groups of one matrix tile
-// on the group kernel (kWideWaves waves per workgroup share a group's pages at
-// head_dim 64, kWaves at 128) than as prefill groups of 64 rows: those read each
-// key once per 64 rows, but put a short launch on few CUs, whose chain of key
-// tiles it then waits for.  Both sides in us per launch, measured on MI355X with
-// 12 heads x 64 (32 x 128), the larger of the longest item's chain and the
-// launch's share of work per CU:
-// * prefill groups: 3 (Q8 3.4), plus 0.55 per 32-key tile of the longest
-//   (head_dim 128: per 16 keys; Q8: 1.15), or 0.39 (Q8 0.57) per tile a CU
-//   receives;
-// * tile groups: 4.6, plus 0.75 per round of the waves over the longest's pages
-//   (head_dim 128: 1.08), or 0.6 per group and 0.115 per page (0.3) a CU
-//   receives.
-// One layer, one prompt, prefill / tile groups: 64 rows 4.3 / 4.7, 320 rows 8.4 /
-// 6.3, 509 rows 12.0 / 8.7, 64 rows after 300 9.3 / 6.8, after 2000 36.9 / 16.2; 2 x
-// 256 rows 7.9 / 7.7, 5 x 256 8.5 / 9.8; Q8 100 rows 7.2 / 5.3, 509 rows 19.3 /
-// 9.6; head_dim 128 256 rows 12.4 / 10.6, 500 rows 21 / 23; 12 layers 100 rows 5.7
-// / 7.6, Q8 500 rows after 300 54 / 74.
-bool small_groups(ni_kv* kv, uint32_t n_lay) {
-    const Plan& P = kv->plan;
-    const auto& qr = kv->qrows;
-    // (a fused or prompt-chunk plan's chunks must run in the prefill launch)
-    if (P.fused || P.seq_prefill) return false;
-    const bool q8 = is_q8(kv->o), d64 = kv->o.head_dim == 64;
-    uint64_t pages = 0, groups = 0, tiles = 0, max_pages = 0;  // of tile groups; 32-key tiles of prefill groups
-    // After prefill groups, the runs' last 1..16 rows are a launch of their
-    // own: on the row kernel, q and the weights in f32, if each is one row
-    // (which as part of a tile group would be f16 pairs), else on the group
-    // kernel.
-    bool last_row = false, last_group = false;
-    for (size_t i = 0; i < qr.size();) {
-        size_t e = i + 1;
-        while (e < qr.size() && qr[e].seq == qr[i].seq && qr[e].row == qr[e - 1].row + 1 && qr[e].pos == qr[e - 1].pos + 1)
-            e++;
-        if (e - i <= kMfmaTile) return false;  // not a launch of prompt chunks only
-        const size_t last = (e - i) % kPrefillRows;
-        last_row |= last == 1;
-        last_group |= last > 1 && last <= kMfmaTile;
-        const uint32_t end = qr[e - 1].pos + 1;
-        for (uint32_t p = qr[i].pos; p < end; p += kMfmaTile, groups++)
-            pages += (std::min(p + kMfmaTile, end) + kPage - 1) / kPage;
-        for (uint32_t p = qr[i].pos; p < end; p += kPrefillRows) tiles += (std::min(p + kPrefillRows, end) + 31) / 32;
-        max_pages = std::max<uint64_t>(max_pages, (end + kPage - 1) / kPage);
-        i = e;
-    }
-    if (last_row && !last_group) return false;
-    const double per_cu = (double)n_lay * kv->o.n_head / device_cus();
-    const double per_tile = q8 ? 1.15 : 0.55, tile_load = q8 ? 0.57 : 0.39;
-    const double chain64 = per_tile * (d64 ? (max_pages + 1) / 2 : max_pages);
-    const double us64 = (q8 ? 3.4 : 3.0) + std::max(chain64, tile_load * (d64 ? 1 : 2) * per_cu * tiles);
-    const uint64_t waves = d64 ? kWideWaves : 4;
-    const double us16 = 4.6 + std::max((d64 ? 0.75 : 1.08) * ((max_pages + waves - 1) / waves),
-                                       per_cu * (0.6 * groups + (d64 ? 0.115 : 0.3) * pages));
-    return us16 < us64;
-}
-
 // Query rows that share a pass over their sequence's keys.
 struct Group {
     uint32_t seq, row0, pos0, nq;
@@ -663,6 +607,85 @@ Cut auto_cut(const ni_kv* kv, const std::vector<Group>& groups, uint32_t n_lay, 
     return fits ? cut : wide;
 }
 
+// Whether a launch of prompt chunks runs faster as groups of one matrix tile
+// (`tiles`, cut by tc) on the group kernel, several waves of a workgroup sharing a
+// group's pages, than as prefill groups of 64 rows (`groups`, cut by gc): those
+// read each key once per 64 rows, but put a short launch on few CUs, whose chain
+// of key tiles it then waits for, and leave a run's last 1..16 rows to a launch
+// of their own.  Both sides in us per launch, measured on MI355X with 12 heads x
+// 64 (32 x 128), the larger of the longest item's chain and the launch's share of
+// work per CU:
+// * prefill groups: 3 (Q8 3.4), plus 0.55 per 32-key tile of the longest
+//   (head_dim 128: per 16 keys; Q8: 1.15), or 0.39 (Q8 0.57) per tile a CU
+//   receives; with a launch of last rows 3 and 0.75 per round of its waves more;
+// * tile groups: 4.6, plus 0.75 per round of the waves over the longest's pages
+//   (head_dim 128: 1.08), or 0.6 per group and 0.115 per page (0.3) a CU
+//   receives;
+// * either, in partitions: 4 and the time of their partials, ~1 per MB, more;
+//   prefill groups' chains 0.35 times longer for every further whole partition
+//   a CU receives.
+// One layer, one prompt, prefill / tile groups: 64 rows 4.3 / 4.7, 320 rows 8.4 /
+// 6.3, 509 rows 12.0 / 8.7, 64 rows after 300 9.3 / 6.8, after 2000 36.9 / 16.2; 2 x
+// 256 rows 7.9 / 7.7, 5 x 256 8.5 / 9.8; Q8 100 rows 7.2 / 5.3, 509 rows 19.3 /
+// 9.6 (attention calls: a step of prompt chunks on a Q8 pool keeps its prefill
+// groups, P.seq_prefill); head_dim 128 250 rows 14.0 / 11.5, 500 rows 21 / 23; 2
+// layers, 64 rows after 500 (partitions) 24.6 / 31.6; 12 layers x 64 200 rows 18.8 /
+// 10.4, 64 rows after 5000 (partitions) 91 / 102, after 9000 111 / 192.
+bool small_groups(const ni_kv* kv, const std::vector<Group>& groups, const Cut& gc, const std::vector<Group>& tiles,
+                  const Cut& tc, uint32_t n_lay) {
+    // (a fused step's chunks must run in the prefill launch, and a Q8 step of
+    // prompt chunks keeps it for its appends)
+    if (kv->plan.fused || kv->plan.seq_prefill) return false;
+    const bool q8 = is_q8(kv->o), d64 = kv->o.head_dim == 64;
+    const double lh = (double)n_lay * kv->o.n_head, per_cu = lh / device_cus();
+    const double mb = lh * (kv->o.head_dim + 2) * sizeof(float) * 1e-6;  // of a slot, per row
+    // Prefill groups.  The runs' last 1..16 rows are a launch of their own: on
+    // the row kernel, q and the weights in f32, if each is one row (which as
+    // part of a tile group would be f16 pairs), else on the group kernel.
+    bool last_row = false, last_group = false;
+    uint32_t chain = 0, last_chain = 0;
+    uint64_t n_tiles = 0, slots = 0, full = 0, last_slots = 0;
+    for (size_t i = 0; i < groups.size(); i++) {
+        const Group& g = groups[i];
+        const uint32_t n = gc.n_parts(g);
+        if (!g.prefill()) {
+            const Group* b = i ? &groups[i - 1] : nullptr;
+            if (!b || b->nq != kPrefillRows || b->seq != g.seq || b->row0 + b->nq != g.row0 || b->keys() != g.pos0)
+                return false;  // not a launch of prompt chunks only
+            (g.nq == 1 ? last_row : last_group) = true;
+            last_chain = std::max(last_chain, std::min(g.keys(), gc.part));
+            last_slots += n > 1 ? n : 0;
+            continue;
+        }
+        chain = std::max(chain, std::min(g.keys(), gc.pre_part));
+        n_tiles += (g.keys() + 31) / 32;
+        slots += n > 1 ? n : 0;
+        full += n > 1 ? g.keys() / gc.pre_part : 0;
+    }
+    if (last_row && !last_group) return false;
+    const double shared = full ? 1 + 0.35 * std::floor(per_cu * full) : 1;
+    double us64 = (q8 ? 3.4 : 3.0) + std::max((q8 ? 1.15 : 0.55) * (d64 ? (chain + 31) / 32 : (chain + 15) / 16) * shared,
+                                              (q8 ? 0.57 : 0.39) * (d64 ? 1 : 2) * per_cu * n_tiles);
+    if (slots) us64 += 4 + mb * kPrefillRows * slots;
+    const double wave = d64 ? 0.75 : 1.08;  // a round of a workgroup's waves over pages
+    auto rounds = [&](uint32_t keys, uint32_t waves) { return (keys + waves * kPage - 1) / (waves * kPage); };
+    if (last_group) us64 += 3 + wave * rounds(last_chain, 4) + (last_slots ? 4 + mb * kMfmaTile * last_slots : 0);
+    // Tile groups.
+    uint64_t pages = 0;
+    chain = 0;
+    slots = 0;
+    for (const Group& g : tiles) {
+        const uint32_t n = tc.n_parts(g);
+        pages += (g.keys() + kPage - 1) / kPage;
+        chain = std::max(chain, std::min(g.keys(), tc.part));
+        slots += n > 1 ? n : 0;
+    }
+    double us16 = 4.6 + std::max(wave * rounds(chain, tc.wide ? kWideWaves : 4),
+                                 per_cu * (0.6 * tiles.size() + (d64 ? 0.115 : 0.3) * pages));
+    if (slots) us16 += 4 + mb * kMfmaTile * slots;
+    return us16 < us64;
+}
+
 // Attention part of a plan: group the query rows, cut each group's keys into
 // partitions, sort the items longest first.
 int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
@@ -686,10 +709,12 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
     Cut cut{split_tokens, split_tokens, 0};
     if (split_tokens == 0) {
         cut = auto_cut(kv, groups, n_lay, n_table);
-        if (prefill && small_groups(kv, n_lay)) {
+        const bool chunks = std::any_of(groups.begin(), groups.end(), [](const Group& g) { return g.prefill(); });
+        if (prefill && chunks) {
             std::vector<Group> tiles = form_groups(qr, max_group_rows(kv));
             const Cut c = auto_cut(kv, tiles, n_lay, n_table);
-            if (noalloc_takes(kv, tiles, c, n_lay, n_table) || !noalloc_takes(kv, groups, cut, n_lay, n_table)) {
+            if (small_groups(kv, groups, cut, tiles, c, n_lay) &&
+                (noalloc_takes(kv, tiles, c, n_lay, n_table) || !noalloc_takes(kv, groups, cut, n_lay, n_table))) {
                 groups.swap(tiles);
                 cut = c;
             }

@@ -74,17 +74,17 @@ def test_same_rows_as_prefill_groups(gpu, q8, n_layer, ctx, rows):
     kv.close()
 
 
-def _prompt(n_layer, ctx, rows, head_dim, g, q8=False):
+def _prompt(n_layer, ctx, rows, head_dim, g, c=768):
     """One sequence of ctx + rows positions, its K/V in the cache, and q for the last `rows`."""
-    n, h = ctx + rows, 768 // head_dim
+    n, h = ctx + rows, c // head_dim
     kv = na.PagedKv(na.BatchOpts(n_layer=n_layer, n_head=h, head_dim=head_dim, kv_blocks=n // 16 + 1, max_seqs=1,
-                                 n_ctx=n, max_rows=n, q8=q8))
+                                 n_ctx=n, max_rows=n))
     s = kv.add_seq()
     kv.reserve(s, n)
-    k, v = (torch.randn((n_layer, n, 768), device="cuda", generator=g).half().float() for _ in range(2))
+    k, v = (torch.randn((n_layer, n, c), device="cuda", generator=g).half().float() for _ in range(2))
     kv.append([(s, i) for i in range(n)], k, v)
     kv.commit(s, n)
-    q = torch.randn((n_layer, rows, 768), device="cuda", generator=g)
+    q = torch.randn((n_layer, rows, c), device="cuda", generator=g)
     return kv, [(s, ctx + i) for i in range(rows)], q, k, v
 
 
@@ -158,3 +158,20 @@ def test_a_split_last_group_fits_the_noalloc_scratch(gpu, rows):
         outs.append(out)
         kv.close()
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("n_layer,head_dim,ctx,rows,tiles", [
+    (1, 64, 0, 509, True), (1, 64, 1300, 64, True), (12, 64, 0, 200, True), (12, 64, 700, 32, True),
+    (12, 64, 0, 512, False), (12, 64, 5000, 64, False), (12, 64, 9000, 64, False), (1, 64, 0, 513, False),
+    (1, 128, 0, 250, True), (1, 128, 1500, 64, True), (2, 128, 500, 64, False), (1, 128, 0, 500, False)], ids=str)
+def test_which_groups_run(gpu, n_layer, head_dim, ctx, rows, tiles):
+    """Prefill groups and tile groups of the same rows differ in rounding, so the
+    bits of a launch with the automatic cut are a prefill launch's (an explicit
+    partition size, as large as the automatic one) exactly where the rule says
+    so: 16-row groups where they are faster with all their launches, the merge
+    of their partitions included."""
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    kv, at, q, _, _ = _prompt(n_layer, ctx, rows, head_dim, g, 768 if head_dim == 64 else 4096)
+    same = torch.equal(kv.attention(q, at), kv.attention(q, at, split_tokens=4096))
+    assert same != tiles
+    kv.close()
