@@ -92,10 +92,12 @@ def _torch():
 
 
 def _stream_ptr(stream) -> int:
-    if stream is None and _raw_stream is not None and _get_device is not None and _tc.cuda.is_initialized():
+    if stream is not None:
+        return int(stream.cuda_stream)
+    torch = _torch()  # (sets the others before _tc: whole for every thread once it returns)
+    if _raw_stream is not None and _get_device is not None and torch.cuda.is_initialized():
         return _raw_stream(_get_device())
-    s = stream if stream is not None else _torch().cuda.current_stream()
-    return int(s.cuda_stream)
+    return int(torch.cuda.current_stream().cuda_stream)
 
 
 def _fits(t, rows, c, device):

@@ -100,3 +100,21 @@ def test_contiguous_attention_shapes():
         na.attention(f(1, C), ok_kv, ok_kv, 2, 3, H, D)  # q one row short
     with pytest.raises(TypeError, match="CUDA"):
         na.attention(ok_q, ok_kv, ok_kv, 2, 3, H, D)  # the right shape, but not on the GPU
+
+
+def test_stream_handle_while_another_thread_sets_up(monkeypatch):
+    """The stream query between the steps of another thread's first call: the
+    handle query already found, torch not yet recorded."""
+    from nanoinfer_amd import batch
+
+    monkeypatch.setattr(batch, "_raw_stream", lambda dev: 7)
+    monkeypatch.setattr(batch, "_get_device", lambda: 0)
+    monkeypatch.setattr(batch, "_tc", None)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: type("S", (), {"cuda_stream": 11})())
+    assert batch._stream_ptr(None) == 11
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(batch, "_raw_stream", lambda dev: 7)
+    monkeypatch.setattr(batch, "_get_device", lambda: 0)
+    assert batch._stream_ptr(None) == 7
+    assert batch._stream_ptr(type("S", (), {"cuda_stream": 13})()) == 13
