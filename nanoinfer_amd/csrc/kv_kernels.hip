@@ -3526,10 +3526,13 @@ hipError_t launch_qkv_t(const QkvLaunch& a, const void* ip, uint32_t ib, hipStre
     // rows f32 23.9 / 21.3, f16 24.0 / 21.0, q4_0 24.9 / 22.3; 640 rows f32 31.5 /
     // 29.7, q4_0 34.9 / 32.1.  One block more loses where it starts a round
     // (480 rows f32 24.8 / 26.7), and below 8 blocks there are too few
-    // workgroups to hide a chunk's loads (224 rows q8_0 13.4 / 13.8).
+    // workgroups to hide a chunk's loads (224 rows q8_0 13.4 / 13.8).  Nor do f32
+    // weights where the CU gets five, a second round of one (16 heads x 64, 416
+    // rows 43.1 / 46.0, 25 heads, 256 rows 63.7 / 67.6; q4_0, whose conversions the
+    // 16-wide tiles repeat, 47.0 / 42.5 and 71.4 / 64.5).
     const uint64_t cus = device_cus();
     auto blocks = [&](uint64_t fb) { return ((uint64_t)row_tiles * (a.n_feat / (16 * fb)) + cus - 1) / cus * fb; };
-    const bool pair = a.n_feat % 32 == 0 && blocks(1) >= 8 && blocks(2) <= blocks(1);
+    const bool pair = a.n_feat % 32 == 0 && blocks(1) >= 8 && blocks(2) <= blocks(1) && (WF != kWF32 || blocks(2) != 10);
     return with_plan(a, ip, ib, [&](auto pa) {
         constexpr int INL = sizeof(pa.b) > 4 ? (int)sizeof(pa.b) : 0;
         if (pair)

@@ -16,9 +16,9 @@ from nanoinfer_amd import workloads
 pytestmark = pytest.mark.gpu
 
 
-# 12 x 64 on 256 CUs: 16-wide up to 384 rows, 32-wide at 385..448, 16-wide at 449, 48-wide at 512, 32-wide at 640;
-# 900 rows leave 4 rows in the last tile.
-@pytest.mark.parametrize("n", [384, 385, 417, 448, 449, 512, 640, 900])
+# 12 x 64 on 256 CUs: 16-wide up to 384 rows, 32-wide at 385..448, 16-wide at 449, 48-wide at 512, 32-wide at 520
+# (f32: 16-wide) and 640; 900 rows leave 4 rows in the last tile.
+@pytest.mark.parametrize("n", [384, 385, 417, 448, 449, 512, 520, 640, 900])
 @pytest.mark.parametrize("fmt", ["f32", "f16", "q8_0", "q4_0"])
 def test_tile_widths_agree(gpu, oracle_lib, n, fmt):
     kv = na.PagedKv(na.BatchOpts(**workloads.GPT2, kv_blocks=8, max_seqs=2, n_ctx=64, max_rows=1024))
