@@ -3617,13 +3617,14 @@ hipError_t launch_attention_rows_t(const RowsLaunch& a, hipStream_t s) {
     // every query reads its keys (12 heads x 64, row against tile kernel: 128
     // queries of 128 keys 4.6 / 5.2 us, 256 of 256 11.4 / 6.9, 64 of 1064 18.2
     // / 16.0, 1024 of 1024 109 / 26; 32 heads x 128: 16 of 1016 27.6 / 38, 32 of
-    // 1032 52 / 40, 250 of 250 49 / 20).  The tile kernel holds 16 rows'
-    // offsets in 32 bits.
+    // 1032 52 / 40, 17 of 3017 88 / 101, 250 of 250 49 / 20; 2 heads x 128: 400 of 900
+    // 30.5 / 32.7, 700 of 700 27.4 / 25.7).  The tile kernel holds 16 rows' offsets
+    // in 32 bits.
     const uint64_t n_kv = (uint64_t)a.q_pos0 + a.n_q;
     const uint64_t keys = (uint64_t)a.n_q * a.q_pos0 + (uint64_t)a.n_q * (a.n_q + 1) / 2;
     const int64_t max_stride = (int64_t)1 << 24;  // floats
     if (a.k_stride <= max_stride && a.v_stride <= max_stride &&
-        (double)keys * a.n_head * D > (D == 64 ? 46000.0 : 66000.0) * (double)(n_kv + 150)) {
+        (double)keys * a.n_head * D > (D == 64 ? 46000.0 : 70000.0) * (double)(n_kv + 150)) {
         const uint32_t blocks = (a.n_q + kRowsTile - 1) / kRowsTile * a.n_head;
         if constexpr (D == 64) {
             // 8 waves while that leaves CUs half empty (384 workgroups: 11.6
