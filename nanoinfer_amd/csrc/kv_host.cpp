@@ -534,6 +534,7 @@ bool noalloc_takes(const ni_kv* kv, const std::vector<Group>& groups, const Cut&
 // 1000 keys of mean (5 rows, 12 layers: 8 x U[64,1000] 27.9 / 25.5, 13 45.1 / 42.0;
 // one of 700 and 3 of 100 9.8 / 12.2, 7 of 100 15.8 / 13.2; one of 2000 and 7 of
 // 100 20.0 / 27.2; one layer, one of 4090 and 159 of 100 32.2 / 50.9).
+//
 // Prefill groups (more rows than one matrix tile, in a launch of their
 // own) are split automatically only past kLongItem keys: each of their
 // workgroups already carries 64 queries, and splitting them to fill the
@@ -629,8 +630,8 @@ Cut auto_cut(const ni_kv* kv, const std::vector<Group>& groups, uint32_t n_lay, 
 // 256 rows 7.9 / 7.7, 5 x 256 8.5 / 9.8; Q8 100 rows 7.2 / 5.3, 509 rows 19.3 /
 // 9.6 (attention calls: a step of prompt chunks on a Q8 pool keeps its prefill
 // groups, P.seq_prefill); head_dim 128 250 rows 14.0 / 11.5, 500 rows 21 / 23; 2
-// layers, 64 rows after 500 (partitions) 24.6 / 31.6; 12 layers x 64 200 rows 18.8 /
-// 10.4, 64 rows after 5000 (partitions) 91 / 102, after 9000 111 / 192.
+// layers, 64 rows after 500 (partitions) 24.6 / 31.6; 12 layers x 64 200 rows 18.7 /
+// 15.6, 64 rows after 5000 (partitions) 91 / 102, after 9000 111 / 192.
 bool small_groups(const ni_kv* kv, const std::vector<Group>& groups, const Cut& gc, const std::vector<Group>& tiles,
                   const Cut& tc, uint32_t n_lay) {
     // (a fused step's chunks must run in the prefill launch, and a Q8 step of
