@@ -2046,8 +2046,9 @@ __device__ __forceinline__ void wait_tiles(uint32_t ahead) {
 // against 109 on attn_rows_kernel, where every query re-reads its keys.  The
 // matrix cores are busy 39% of it: the accumulators take 196 VGPRs at head_dim
 // 64, two waves per SIMD (128: 256 and 119 AGPRs, one), too few to hide the
-// chain, and 768 workgroups are 1.5 rounds of the two per CU.  32 queries per wave (K/V read half as often, half the workgroups) took 28-34
-// us, all of K and V through LDS 27, more keys in flight (8 waves) 29.
+// chain, and 768 workgroups are 1.5 rounds of the two per CU.  32 queries per
+// wave (K/V read half as often, half the workgroups) took 28-34 us, all of K and
+// V through LDS 27, more keys in flight (8 waves) 29.
 //
 // Error: the sums are cut so that it is that of attn_rows_kernel (1.3e-7 of
 // the result against 64 bits at 1024 keys; one accumulator throughout 2.6e-7):

@@ -310,6 +310,40 @@ def test_noalloc_step_replayed_from_a_graph(gpu):
     b.close()
 
 
+def test_noalloc_prompt_replayed_from_a_graph(gpu):
+    """A prompt on 16-row groups (one layer, 509 rows, the automatic cut) and a
+    decode step of few units (whole workgroups), captured and replayed."""
+    L, H, D = 1, 12, 64
+    C_ = H * D
+    opts = na.BatchOpts(n_layer=L, n_head=H, head_dim=D, kv_blocks=128, max_seqs=4, n_ctx=1024, max_rows=512)
+    lib = _abi.lib()
+    g = torch.Generator(device="cuda").manual_seed(83)
+    for work, lens in (([(0, 509, 509)], [3]), ([(0, 1, 1), (1, 1, 1)], [700, 150])):
+        a, b = na.PagedKv(opts), na.PagedKv(opts)
+        seqs = list(range(len(lens)))
+        fill([a, b], seqs, lens, g, C_)
+        n = sum(w[1] for w in work)
+        q, k, v = (torch.randn((L, n, C_), device="cuda", generator=g) for _ in range(3))
+        out_a, out_b = (torch.full((L, n, C_), float("nan"), device="cuda") for _ in range(2))
+        assert call(a, lib.ni_kv_step, work, q, k, v, out_a, 0) == 0, lib.ni_kv_last_error(a.handle).decode()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        say(f"graph: capturing {n} rows")
+        with torch.cuda.graph(graph):
+            rc = call(b, lib.ni_kv_step_noalloc, work, q, k, v, out_b, 0)
+        assert rc == 0, lib.ni_kv_last_error(b.handle).decode()
+        for rep in range(3):
+            out_b.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out_a, out_b), f"replay {rep + 1}"
+            same_state(a, b, seqs)  # eager gathers between the replays
+        del graph
+        a.close()
+        b.close()
+
+
 def test_noalloc_scratch_held_by_one_handle(gpu):
     """The GPU's one scratch array belongs to the first handle that calls
     ni_kv_step_noalloc: another handle's call is refused (nothing launched,
