@@ -89,8 +89,8 @@ struct Plan {
     std::vector<AppendEntry> orphans;  // fused: rows of sequences without queries
     std::vector<AttnItem> items;
     std::vector<MergeItem> merges;
-    std::vector<AttnItem> pitems;    // prefill groups (attn_prefill_kernel), their merges
-    std::vector<MergeItem> pmerges;  //   and partial slots (a region after the others')
+    std::vector<AttnItem> pitems;    // prefill groups (attn_prefill_kernel; pre_tile 1: single rows beside tile
+    std::vector<MergeItem> pmerges;  //   groups), their merges and partial slots (a region after the others')
     std::vector<uint32_t> table;
     std::vector<PrefillSeq> pseqs;  // prompt-chunk step: the prefill launch appends, a workgroup per sequence
     std::vector<uint16_t> order;    // balanced wide launch: the (item, layer, head) unit of each workgroup
@@ -101,6 +101,7 @@ struct Plan {
     uint32_t napp_total = 0;  // fused: rows the attention items append
     bool fused = false;
     uint32_t wide = 0;        // waves per attention workgroup: AttnLaunch::wide
+    uint32_t pre_tile = kPrefillRows, pre_wide = 0;  // AttnLaunch::nq_tile and wide of the pitems' launch
     bool seq_prefill = false; // every row belongs to a sequence queried as prefill groups (see pseqs)
     // Some launch of the plan reads the append entries `app` (an append
     // launch, a workgroup prologue, a prefill workgroup's appends); a fused
@@ -125,6 +126,8 @@ struct Plan {
         napp_total = 0;
         fused = false;
         wide = 0;
+        pre_tile = kPrefillRows;
+        pre_wide = 0;
         app_read = true;
     }
 };
@@ -427,7 +430,7 @@ void balance_prefill_units(Plan& P, uint32_t n_lay, uint32_t n_head, uint64_t C,
 struct Group {
     uint32_t seq, row0, pos0, nq;
     uint32_t new_begin, new_end, app_first;
-    uint32_t pre;  // runs in the prefill launch whatever its size
+    uint32_t pre;  // runs in the prefill launch (Cut::pre_tile) whatever its size
     uint32_t keys() const { return pos0 + nq; }
     bool prefill() const { return pre || nq > kMfmaTile; }
 };
@@ -450,11 +453,12 @@ std::vector<Group> form_groups(const std::vector<QRow>& qr, uint32_t max_rows) {
     return groups;
 }
 
-// How a launch cuts its groups: keys per partition, of groups of up to one
-// matrix tile and of prefill groups, and the former's workgroups
-// (AttnLaunch::wide).
+// How a launch cuts its groups: keys per partition and workgroups
+// (AttnLaunch::wide) of groups of up to one matrix tile, and of the prefill
+// launch's, whose rows per group at most are pre_tile.
 struct Cut {
     uint32_t part, pre_part, wide;
+    uint32_t pre_tile = kPrefillRows, pre_wide = 0;
     uint32_t n_parts(const Group& g) const {
         const uint32_t p = g.prefill() ? pre_part : part;
         return (g.keys() + p - 1) / p;
@@ -492,7 +496,7 @@ bool noalloc_takes(const ni_kv* kv, const std::vector<Group>& groups, const Cut&
     add(n_table, sizeof(uint32_t));
     const uint64_t units = items[0] * lh;
     if (cut.wide && units > device_cus() && (nq_tile > 1 || units >= 512)) add(units, sizeof(uint16_t));  // their order
-    const size_t partials = (slots[0] * nq_tile + slots[1] * kPrefillRows) * lh * (kv->o.head_dim + 2) * sizeof(float);
+    const size_t partials = (slots[0] * nq_tile + slots[1] * cut.pre_tile) * lh * (kv->o.head_dim + 2) * sizeof(float);
     return bytes <= kInlinePlanBytes && partials <= kScratchBytes;
 }
 
@@ -640,10 +644,10 @@ bool small_groups(const ni_kv* kv, const std::vector<Group>& groups, const Cut& 
     const bool q8 = is_q8(kv->o), d64 = kv->o.head_dim == 64;
     const double lh = (double)n_lay * kv->o.n_head, per_cu = lh / device_cus();
     const double mb = lh * (kv->o.head_dim + 2) * sizeof(float) * 1e-6;  // of a slot, per row
-    // Prefill groups.  The runs' last 1..16 rows are a launch of their own: on
-    // the row kernel, q and the weights in f32, if each is one row (which as
-    // part of a tile group would be f16 pairs), else on the group kernel.
-    bool last_row = false, last_group = false;
+    // Prefill groups.  The runs' last 1..16 rows are a launch of their own, on
+    // the group kernel, or the row kernel if each is one row: then the tile
+    // groups have that launch beside them too (plan_attention).
+    bool last_group = false;
     uint32_t chain = 0, last_chain = 0;
     uint64_t n_tiles = 0, slots = 0, full = 0, last_slots = 0;
     for (size_t i = 0; i < groups.size(); i++) {
@@ -653,7 +657,7 @@ bool small_groups(const ni_kv* kv, const std::vector<Group>& groups, const Cut& 
             const Group* b = i ? &groups[i - 1] : nullptr;
             if (!b || b->nq != kPrefillRows || b->seq != g.seq || b->row0 + b->nq != g.row0 || b->keys() != g.pos0)
                 return false;  // not a launch of prompt chunks only
-            (g.nq == 1 ? last_row : last_group) = true;
+            last_group |= g.nq > 1;
             last_chain = std::max(last_chain, std::min(g.keys(), gc.part));
             last_slots += n > 1 ? n : 0;
             continue;
@@ -663,7 +667,6 @@ bool small_groups(const ni_kv* kv, const std::vector<Group>& groups, const Cut& 
         slots += n > 1 ? n : 0;
         full += n > 1 ? g.keys() / gc.pre_part : 0;
     }
-    if (last_row && !last_group) return false;
     const double shared = full ? 1 + 0.35 * std::floor(per_cu * full) : 1;
     double us64 = (q8 ? 3.4 : 3.0) + std::max((q8 ? 1.15 : 0.55) * (d64 ? (chain + 31) / 32 : (chain + 15) / 16) * shared,
                                               (q8 ? 0.57 : 0.39) * (d64 ? 1 : 2) * per_cu * n_tiles);
@@ -712,16 +715,37 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
         cut = auto_cut(kv, groups, n_lay, n_table);
         const bool chunks = std::any_of(groups.begin(), groups.end(), [](const Group& g) { return g.prefill(); });
         if (prefill && chunks) {
-            std::vector<Group> tiles = form_groups(qr, max_group_rows(kv));
-            const Cut c = auto_cut(kv, tiles, n_lay, n_table);
-            if (small_groups(kv, groups, cut, tiles, c, n_lay) &&
-                (noalloc_takes(kv, tiles, c, n_lay, n_table) || !noalloc_takes(kv, groups, cut, n_lay, n_table))) {
-                groups.swap(tiles);
-                cut = c;
+            std::vector<Group> tiles = form_groups(qr, max_group_rows(kv)), rows;
+            // After prefill groups, single last rows run on the row kernel, q
+            // and the weights in f32.  Beside tile groups they keep a launch on
+            // it (as part of the groups' they would be f16 pairs).
+            uint32_t last_nq = 0;  // rows of the largest group outside the prefill launch
+            for (const Group& g : groups) last_nq = std::max(last_nq, g.prefill() ? 0u : g.nq);
+            if (last_nq == 1) {
+                const auto single = std::stable_partition(tiles.begin(), tiles.end(), [](const Group& g) { return g.nq > 1; });
+                rows.assign(single, tiles.end());
+                tiles.erase(single, tiles.end());
+            }
+            Cut c = auto_cut(kv, tiles, n_lay, n_table);
+            if (!rows.empty()) {
+                const Cut r = auto_cut(kv, rows, n_lay, n_table);
+                c.pre_tile = 1;
+                c.pre_part = r.part;
+                c.pre_wide = r.wide;
+                for (Group& g : rows) g.pre = 1;
+            }
+            if (small_groups(kv, groups, cut, tiles, c, n_lay)) {
+                tiles.insert(tiles.end(), rows.begin(), rows.end());
+                if (noalloc_takes(kv, tiles, c, n_lay, n_table) || !noalloc_takes(kv, groups, cut, n_lay, n_table)) {
+                    groups.swap(tiles);
+                    cut = c;
+                }
             }
         }
     }
     P.wide = cut.wide;
+    P.pre_tile = cut.pre_tile;
+    P.pre_wide = cut.pre_wide;
     for (const Group& g : groups) {
         if (kv->seq_tab[g.seq] >= 0) continue;
         kv->seq_tab[g.seq] = (int64_t)P.table.size();
@@ -849,7 +873,7 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
     // f16 prefill items carry their first pages' ids (the prefill kernel
     // issues its first tiles' DMA from them, beside the item's q and page-id
     // loads instead of after them).
-    if (!is_q8(kv->o)) {
+    if (!is_q8(kv->o) && P.pre_tile == kPrefillRows) {
         for (AttnItem& it : P.pitems) {
             const uint32_t pb = it.kv_begin / kPage, pe = (it.kv_end + kPage - 1) / kPage;
             for (uint32_t i = 0; i < 4; i++) it.first_pages[i] = pe > pb ? P.table[it.tab + std::min(pb + i, pe - 1)] : 0u;
@@ -1125,7 +1149,7 @@ int run_placed(ni_kv* kv, const Plan& P, const Offsets& off, const PlanRef& ref,
     const uint32_t D = kv->o.head_dim, H = kv->o.n_head;
     // Partials: the single-row/group launch's slots, then the prefill launch's.
     const size_t main_floats = (size_t)P.n_slots * n_lay * H * P.nq_tile * (D + 2);
-    const size_t pre_floats = (size_t)P.n_pslots * n_lay * H * kPrefillRows * (D + 2);
+    const size_t pre_floats = (size_t)P.n_pslots * n_lay * H * P.pre_tile * (D + 2);
     float* partials = nullptr;
     if (main_floats + pre_floats > 0) {
         int rc = ensure_partials(kv, (main_floats + pre_floats) * sizeof(float), s, &partials);
@@ -1192,8 +1216,9 @@ int run_placed(ni_kv* kv, const Plan& P, const Offsets& off, const PlanRef& ref,
         }
     }
     if (!P.pitems.empty()) {
-        // Prefill groups: their own launch (after the append above), items,
-        // merges and partials region; never fused.
+        // Prefill groups (or single rows beside tile groups): their own launch
+        // (after the append above), items, merges and partials region; never
+        // fused.
         AttnLaunch a{};
         a.pool = kv->geom();
         a.q = q;
@@ -1211,7 +1236,8 @@ int run_placed(ni_kv* kv, const Plan& P, const Offsets& off, const PlanRef& ref,
         a.n_merges = (uint32_t)P.pmerges.size();
         a.layer0 = layer0;
         a.n_lay = n_lay;
-        a.nq_tile = kPrefillRows;
+        a.nq_tile = P.pre_tile;
+        a.wide = P.pre_wide;
         a.off_order = (uint32_t)off.porder;
         a.ordered = P.porder.empty() ? 0u : 1u;
         a.qscale = (float)(1.4426950408889634 / std::sqrt((double)D));

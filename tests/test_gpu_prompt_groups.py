@@ -162,14 +162,14 @@ def test_a_split_last_group_fits_the_noalloc_scratch(gpu, rows):
 
 @pytest.mark.parametrize("n_layer,head_dim,ctx,rows,tiles", [
     (1, 64, 0, 509, True), (1, 64, 1300, 64, True), (12, 64, 0, 200, True), (12, 64, 700, 32, True),
-    (12, 64, 0, 512, False), (12, 64, 5000, 64, False), (12, 64, 9000, 64, False), (1, 64, 0, 513, False),
+    (12, 64, 0, 512, False), (12, 64, 5000, 64, False), (12, 64, 9000, 64, False), (1, 64, 0, 513, True),
     (1, 128, 0, 250, True), (1, 128, 1500, 64, True), (2, 128, 500, 64, False), (1, 128, 0, 500, False)], ids=str)
 def test_which_groups_run(gpu, n_layer, head_dim, ctx, rows, tiles):
     """Prefill groups and tile groups of the same rows differ in rounding, so the
     bits of a launch with the automatic cut are a prefill launch's (an explicit
     partition size, as large as the automatic one) exactly where the rule says
     so: 16-row groups where they are faster with all their launches, the merge
-    of their partitions included."""
+    of their partitions and the row launch of a single last row included."""
     g = torch.Generator(device="cuda").manual_seed(rows)
     kv, at, q, _, _ = _prompt(n_layer, ctx, rows, head_dim, g, 768 if head_dim == 64 else 4096)
     same = torch.equal(kv.attention(q, at), kv.attention(q, at, split_tokens=4096))

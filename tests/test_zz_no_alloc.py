@@ -154,7 +154,8 @@ def test_noalloc_q8_prompt_chunks_appended_by_the_prefill_launch(gpu):
 # (n_layer, head_dim, contexts, rows): prompt chunks with the automatic cut.  The last is 27 prompts of 64 rows, one
 # after a long context: as 16-row groups its plan would be past 32 KB, as 64-row groups it is not.
 PROMPTS = [(1, 64, [0], [100]), (1, 64, [0], [509]), (12, 64, [0], [64]), (12, 64, [300], [40]), (2, 64, [0, 70], [200, 90]),
-           (12, 64, [0], [200]), (1, 128, [0], [250]), (2, 128, [500], [64]), (1, 64, [2000], [80]),
+           (12, 64, [0], [200]), (1, 64, [0], [513]), (1, 64, [5000, 0], [65, 129]), (1, 128, [1500], [65]),
+           (1, 128, [0], [250]), (2, 128, [500], [64]), (1, 64, [2000], [80]),
            (1, 64, [4000] + [0] * 26, [64] * 27)]
 
 
