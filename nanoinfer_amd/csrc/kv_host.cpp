@@ -612,6 +612,27 @@ Cut auto_cut(const ni_kv* kv, const std::vector<Group>& groups, uint32_t n_lay, 
     return fits ? cut : wide;
 }
 
+// What bounds a launch of prefill groups, in us (measured: see small_groups).
+struct PrefillUs {
+    double chain, load;  // the longest group's chain of tiles, the launch's tiles per CU
+};
+
+PrefillUs prefill_us(const ni_kv* kv, const std::vector<Group>& groups, const Cut& gc, uint32_t n_lay) {
+    const bool q8 = is_q8(kv->o), d64 = kv->o.head_dim == 64;
+    const double per_cu = (double)n_lay * kv->o.n_head / device_cus();
+    uint32_t chain = 0;
+    uint64_t n_tiles = 0, full = 0;
+    for (const Group& g : groups) {
+        if (!g.prefill()) continue;
+        chain = std::max(chain, std::min(g.keys(), gc.pre_part));
+        n_tiles += (g.keys() + 31) / 32;
+        full += g.keys() > gc.pre_part ? g.keys() / gc.pre_part : 0;
+    }
+    const double shared = full ? 1 + 0.35 * std::floor(per_cu * full) : 1;
+    return {(q8 ? 1.15 : 0.55) * (d64 ? (chain + 31) / 32 : (chain + 15) / 16) * shared,
+            (q8 ? 0.57 : 0.39) * (d64 ? 1 : 2) * per_cu * n_tiles};
+}
+
 // Whether a launch of prompt chunks runs faster as groups of one matrix tile
 // (`tiles`, cut by tc) on the group kernel, several waves of a workgroup sharing a
 // group's pages, than as prefill groups of 64 rows (`groups`, cut by gc): those
@@ -638,9 +659,6 @@ Cut auto_cut(const ni_kv* kv, const std::vector<Group>& groups, uint32_t n_lay, 
 // 15.6, 64 rows after 5000 (partitions) 91 / 102, after 9000 111 / 192.
 bool small_groups(const ni_kv* kv, const std::vector<Group>& groups, const Cut& gc, const std::vector<Group>& tiles,
                   const Cut& tc, uint32_t n_lay) {
-    // (a fused step's chunks must run in the prefill launch, and a Q8 step of
-    // prompt chunks keeps it for its appends)
-    if (kv->plan.fused || kv->plan.seq_prefill) return false;
     const bool q8 = is_q8(kv->o), d64 = kv->o.head_dim == 64;
     const double lh = (double)n_lay * kv->o.n_head, per_cu = lh / device_cus();
     const double mb = lh * (kv->o.head_dim + 2) * sizeof(float) * 1e-6;  // of a slot, per row
@@ -648,8 +666,8 @@ bool small_groups(const ni_kv* kv, const std::vector<Group>& groups, const Cut& 
     // the group kernel, or the row kernel if each is one row: then the tile
     // groups have that launch beside them too (plan_attention).
     bool last_group = false;
-    uint32_t chain = 0, last_chain = 0;
-    uint64_t n_tiles = 0, slots = 0, full = 0, last_slots = 0;
+    uint32_t last_chain = 0;
+    uint64_t slots = 0, last_slots = 0;
     for (size_t i = 0; i < groups.size(); i++) {
         const Group& g = groups[i];
         const uint32_t n = gc.n_parts(g);
@@ -662,21 +680,17 @@ bool small_groups(const ni_kv* kv, const std::vector<Group>& groups, const Cut& 
             last_slots += n > 1 ? n : 0;
             continue;
         }
-        chain = std::max(chain, std::min(g.keys(), gc.pre_part));
-        n_tiles += (g.keys() + 31) / 32;
         slots += n > 1 ? n : 0;
-        full += n > 1 ? g.keys() / gc.pre_part : 0;
     }
-    const double shared = full ? 1 + 0.35 * std::floor(per_cu * full) : 1;
-    double us64 = (q8 ? 3.4 : 3.0) + std::max((q8 ? 1.15 : 0.55) * (d64 ? (chain + 31) / 32 : (chain + 15) / 16) * shared,
-                                              (q8 ? 0.57 : 0.39) * (d64 ? 1 : 2) * per_cu * n_tiles);
+    const PrefillUs pre = prefill_us(kv, groups, gc, n_lay);
+    double us64 = (q8 ? 3.4 : 3.0) + std::max(pre.chain, pre.load);
     if (slots) us64 += 4 + mb * kPrefillRows * slots;
     const double wave = d64 ? 0.75 : 1.08;  // a round of a workgroup's waves over pages
     auto rounds = [&](uint32_t keys, uint32_t waves) { return (keys + waves * kPage - 1) / (waves * kPage); };
     if (last_group) us64 += 3 + wave * rounds(last_chain, 4) + (last_slots ? 4 + mb * kMfmaTile * last_slots : 0);
     // Tile groups.
     uint64_t pages = 0;
-    chain = 0;
+    uint32_t chain = 0;
     slots = 0;
     for (const Group& g : tiles) {
         const uint32_t n = tc.n_parts(g);
@@ -713,8 +727,12 @@ int plan_attention(ni_kv* kv, uint32_t split_tokens, uint32_t n_lay) {
     Cut cut{split_tokens, split_tokens, 0};
     if (split_tokens == 0) {
         cut = auto_cut(kv, groups, n_lay, n_table);
-        const bool chunks = std::any_of(groups.begin(), groups.end(), [](const Group& g) { return g.prefill(); });
-        if (prefill && chunks) {
+        // Prompt chunks as tile groups: not in a fused step, whose chunks must
+        // run in the prefill launch, nor a Q8 step of prompt chunks, which keeps
+        // it for its appends, nor where prefill groups keep the CUs busy anyway
+        // (tile groups take over twice the work).
+        const PrefillUs pre = prefill_us(kv, groups, cut, n_lay);
+        if (prefill && !P.fused && !P.seq_prefill && pre.load < 2 * pre.chain) {
             std::vector<Group> tiles = form_groups(qr, max_group_rows(kv)), rows;
             // After prefill groups, single last rows run on the row kernel, q
             // and the weights in f32.  Beside tile groups they keep a launch on
